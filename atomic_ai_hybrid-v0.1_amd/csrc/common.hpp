@@ -39,15 +39,18 @@ template <> __device__ __forceinline__ float from_f<float>(float x) { return x; 
 template <> __device__ __forceinline__ bf16 from_f<bf16>(float x) { return (bf16)x; }
 
 // jnp.nan_to_num(x, nan=0, posinf=c, neginf=-c): finite values pass unchanged.
+// Selects only: written with early returns this compiled to two nested
+// exec-masked branches per element (GDN2 forward + backward at B4 T8192 H16
+// K = V = 128: 2.11 ms, with the selects 2.02 ms).
 __device__ __forceinline__ float n2n(float x, float c = kClipAcc) {
-  if (__builtin_isnan(x)) return 0.f;
-  if (__builtin_isinf(x)) return x > 0.f ? c : -c;
-  return x;
+  const float y = __builtin_isnan(x) ? 0.f : x;
+  return __builtin_isinf(y) ? __builtin_copysignf(c, y) : y;
 }
-// clip to [-c, c] then nan_to_num.
+// clip to [-c, c] then nan_to_num (v_med3 clips; it returns -c for a NaN,
+// which the select replaces).
 __device__ __forceinline__ float sanitize(float x, float c = kClipAcc) {
-  if (__builtin_isnan(x)) return 0.f;
-  return fminf(fmaxf(x, -c), c);
+  const float y = __builtin_amdgcn_fmed3f(x, -c, c);
+  return __builtin_isnan(x) ? 0.f : y;
 }
 
 // ---------------------------------------------------------------- vector I/O
