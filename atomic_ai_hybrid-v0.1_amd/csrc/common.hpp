@@ -249,6 +249,34 @@ template <> struct Raw8<float> {
   }
 };
 
+// ------------------------------------------------- global memory -> LDS
+// The s_waitcnt immediate that lets at most n vector-memory operations be
+// outstanding (and waits for nothing else).
+constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+// 16 bytes from each lane's global address to 1 KB of LDS at dst (wave-uniform)
+// in lane order, without passing through registers.  Counts in vmcnt.  The
+// wave that issues these waits for them itself (__builtin_amdgcn_s_waitcnt of
+// vmcnt_imm) before the barrier that publishes them.
+__device__ __forceinline__ void dma16(const void* src, void* dst) {
+  typedef const __attribute__((address_space(1))) uint32_t* gp;
+  typedef __attribute__((address_space(3))) uint32_t* lp;
+  __builtin_amdgcn_global_load_lds((gp)(uintptr_t)src, (lp)(uint32_t)(uintptr_t)dst, 16, 0, 0);
+}
+// One dword per lane to LDS nobody reads: brings the lanes' cache lines into L2.
+__device__ __forceinline__ void dma_touch(const void* src, void* dst) {
+  typedef const __attribute__((address_space(1))) uint32_t* gp;
+  typedef __attribute__((address_space(3))) uint32_t* lp;
+  __builtin_amdgcn_global_load_lds((gp)(uintptr_t)src, (lp)(uint32_t)(uintptr_t)dst, 4, 0, 0);
+}
+// A workgroup barrier that does not wait for the wave's own outstanding memory
+// operations (a loader wave keeps its loads in flight across it).
+__device__ __forceinline__ void bare_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Row padding (elements) that keeps rows 16-byte aligned.
 template <typename T> struct Pad { static constexpr int v = 16 / sizeof(T); };
 

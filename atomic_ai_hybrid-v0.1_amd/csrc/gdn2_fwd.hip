@@ -20,7 +20,7 @@
 //   (kernel_d_pipeline.py:94-124): v_new = u - w_pseudo h;
 //   o = scale qg h + Aqk v_new; h = sanitize(h e^{gc_last} + kg^T v_new).
 //   The fp32 state lives in MFMA accumulators for the whole sequence.
-#include "gdn2.hpp"
+#include "gdn2_seq.hpp"
 
 namespace ah {
 
@@ -528,295 +528,488 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
 }
 
 // ------------------------------------------------------------------ state
-template <typename T, int C, int K, int V, int VT>
-struct StateLds {
-  static constexpr int PAD = Pad<T>::v;
-  static constexpr int LK = K + PAD, LC = C + PAD, LU = VT + PAD;
-  // one chunk's staged operands (offsets within a stage buffer)
-  static constexpr int s_w = 0;
-  static constexpr int s_q = s_w + C * LK * (int)sizeof(T);
-  static constexpr int s_kg = s_q + C * LK * (int)sizeof(T);
-  static constexpr int s_aqk = s_kg + C * LK * (int)sizeof(T);
-  static constexpr int s_u = s_aqk + C * LC * (int)sizeof(T);
-  static constexpr int s_gl = s_u + C * LU * (int)sizeof(T);
-  static constexpr int SB = (s_gl + K * 4 + 15) / 16 * 16;
-  static constexpr int REST = VT * LK * (int)sizeof(T) + VT * LC * (int)sizeof(T);
-  // two stage buffers when they fit: chunk n + 1 is written while chunk n
-  // computes, which also saves a barrier per chunk
-  static constexpr int NBUF = 2 * SB + REST <= 160 * 1024 ? 2 : 1;
-  static constexpr int off_ht = NBUF * SB;
-  static constexpr int off_vn = off_ht + VT * LK * (int)sizeof(T);
-  static constexpr int total = off_vn + VT * LC * (int)sizeof(T);
-};
-
 // gdn2_fwd_state mode bits: keep the per-chunk states and v_new for the
 // backward; write o per chunk ([B][H][NT][C][V], the layout of
 // gdn2_inter_chunk_combine's result, kernel_d_pipeline.py:94-124) instead of
 // [B][T][H][V]; sanitise h0 (nan_to_num(clip(h0, +-1e4)), its _sanitize_h0).
 enum { kStateSave = 1, kStateChunkO = 2, kStateSanitizeH0 = 4 };
 
-// NW waves (NW / 4 per SIMD): the state tiles and the [w; q] h tiles of one
-// V tile split over them by row blocks.  PD register sets of chunk operands
-// are in flight (two at eight waves; one at sixteen, where the other waves
-// hide the load latency and the VGPR budget is 128).  With DO, each step's o
-// tiles stay in registers and are written by the next step between its
-// commit and its prefetch (faster with 16-column tiles, slower with 32).
-template <typename T, int C, int K, int V, int VT, int NW = 8, int PD = 2, bool DO = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void gdn2_fwd_state(Gdn2Dims dm, Gdn2Chunks<T> ck,
-                                                     const float* __restrict__ h0, float* __restrict__ o,
-                                                     float* __restrict__ h_final, int mode) {
-  const int save = mode & kStateSave;
-  typedef StateLds<T, C, K, V, VT> L;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[L::total];
-  T* sHt = reinterpret_cast<T*>(lds + L::off_ht);
-  T* sVn = reinterpret_cast<T*>(lds + L::off_vn);
-  // the stage buffer the current chunk reads
-  T *sW, *sQ, *sKg, *sAqk, *sU;
-  float* sGl;
-  auto use_buf = [&](int bsel) {
-    unsigned char* bp = lds + bsel * L::SB;
-    sW = reinterpret_cast<T*>(bp + L::s_w);
-    sQ = reinterpret_cast<T*>(bp + L::s_q);
-    sKg = reinterpret_cast<T*>(bp + L::s_kg);
-    sAqk = reinterpret_cast<T*>(bp + L::s_aqk);
-    sU = reinterpret_cast<T*>(bp + L::s_u);
-    sGl = reinterpret_cast<float*>(bp + L::s_gl);
-  };
-  use_buf(0);
+template <int C, int K, int VT>
+struct StateLds {
+  static constexpr int RB = K * 2, CB = C * 2, UB = VT * 2;  // row bytes
+  // read before a step's first barrier only: two buffers
+  static constexpr int s_w = 0, s_q = C * RB, s_u = 2 * C * RB, s_gl = s_u + C * UB;
+  static constexpr int WQ = s_gl + K * 4;
+  // loaded at the start of a step: three buffers
+  static constexpr int s_kg = 0, s_a = C * RB;
+  static constexpr int KA = C * RB + C * CB;
+  static constexpr int off_wq = 0, off_ka = 2 * WQ, off_h = off_ka + 3 * KA;
+  static constexpr int off_vn = off_h + K * UB;
+  static constexpr int off_pf = off_vn + C * UB;  // where the prefetch wave's loads land
+  static constexpr int total = off_pf + 256;
+  static_assert(total <= 160 * 1024, "one workgroup per CU");
+};
 
-  constexpr int NVT = V / VT;
+// bf16 state loop of one (batch, head, VT columns): waves 0-3 compute v_new
+// and the state, 4-7 o (and store the saves), the next NL load the chunks (see
+// gdn2_seq.hpp), and one more, when launched, touches the lines of the chunk
+// kPrefetch steps on: it hides the memory latency that two chunks in flight do
+// not cover.
+// v_new and the state are computed transposed (columns of h as MFMA rows), so
+// a lane's four results are four consecutive columns of one row of the LDS
+// copies.  Bound by the step's chain of LDS reads, MFMAs and two barriers when
+// the operands come from L2 (0.87 us a chunk at 16 columns, 1.3 at 32, K =
+// 128; the former kernel, in which every wave loaded, staged and computed,
+// 1.40 and 1.7), and by HBM with 256 workgroups and the saves.
+// B1 T32768 H16: 0.825 -> 0.490 ms; B8 T4096 H6 with saves 0.175 -> 0.156 ms;
+// B4 T8192 H16 0.311 -> 0.248 ms, with saves 0.372 -> 0.348 ms; K = 64, B2
+// T4096 H16: 0.083 -> 0.038 ms.
+template <int C, int K, int V, int VT, int NL>
+__global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
+    Gdn2Dims dm, Gdn2Chunks<bf16> ck, const float* __restrict__ h0, float* __restrict__ o,
+    float* __restrict__ h_final, int mode) {
+  typedef StateLds<C, K, VT> L;
+  typedef Mma<bf16> M;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[L::total];
+  constexpr int NVT = V / VT, NTI = VT / 16, RB = K / 64, XK = K / 32, XC = C / 32, PK = K / 8;
+  static_assert(C == 64 && K % 64 == 0, "four row blocks");
+  constexpr int kPrefetch = 4;
   int bh, vt;
   xcd_group_map(blockIdx.x, dm.B * dm.H, NVT, bh, vt);
   const int h = bh % dm.H, bb = bh / dm.H;
   const int v0 = vt * VT;
-  const int wv_id = wave_id();
+  const int wid = wave_id(), w = wid & 3, lane = lane_id(), r16 = lane & 15, g4 = lane >> 4;
+  const size_t bh0 = (size_t)bh * dm.NT;
+  const int last = dm.NT - 1;
+  unsigned char* sH = lds + L::off_h;
+  unsigned char* sVn = lds + L::off_vn;
 
-  // state tiles h[d][v]: (K/16) x (VT/16), TPW per wave
-  constexpr int NTHR = 64 * NW;
-  constexpr int NTI = VT / 16;
-  constexpr int NTH = (K / 16) * NTI;
-  constexpr int TPW = NTH / NW;
-  static_assert(NTH % NW == 0 && TPW >= 1, "state tiles must split evenly over the waves");
-  f32x4 hs[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int tile = wv_id * TPW + t, mi = tile / NTI, ni = tile % NTI;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * mi + tile_row(i), vv = v0 + 16 * ni + tile_col();
-      const float hv = h0 ? h0[((size_t)bh * K + d) * V + vv] : 0.f;
-      hs[t][i] = (mode & kStateSanitizeH0) ? sanitize(hv) : hv;
+  if (wid == 8 + NL) {
+    // ---------------- L2 prefetch: the V tiles of a head share an XCD and split its lines
+    auto prefetch = [&](int n) {
+      if (n > last) return;
+      auto part = [&](const void* p, int bytes) { touch_lines(p, bytes, NVT, vt, lds + L::off_pf); };
+      part(ck.wt + (bh0 + n) * (C * K), C * K * 2);
+      part(ck.qg + (bh0 + n) * (C * K), C * K * 2);
+      part(ck.kg + (bh0 + n) * (C * K), C * K * 2);
+      part(ck.aqk + (bh0 + n) * (C * C), C * C * 2);
+      part(ck.u + (bh0 + n) * (C * V), C * V * 2);
+    };
+    for (int n = 2; n < kPrefetch; ++n) prefetch(n);
+    bare_barrier();
+    for (int n = 0; n < dm.NT; ++n) {
+      prefetch(n + kPrefetch);
+      bare_barrier();
+      bare_barrier();
     }
-    store_tile_t(sHt, L::LK, 16 * mi, 16 * ni, hs[t]);
+    return;
+  }
+  if (wid >= 8) {
+    // ---------------- loader waves
+    const int lw = wid - 8;
+    auto issue_ka = [&](int n) {
+      unsigned char* b = lds + L::off_ka + (n % 3) * L::KA;
+      dma_rows<K, NL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
+      dma_rows<C, NL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
+    };
+    auto issue_wq = [&](int n) {
+      unsigned char* b = lds + L::off_wq + (n & 1) * L::WQ;
+      dma_rows<K, NL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
+      dma_rows<K, NL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
+      // u and gc_last: every wave issues the same number of instructions (it
+      // counts them below), so a wave past the last piece repeats one
+      constexpr int NI = C * L::UB / 1024, PU = VT / 8;
+      static_assert(NI <= NL, "a wave loads one piece of u");
+      const int ins = lw % NI, row = ins * (64 / PU) + lane / PU;
+      dma16(ck.u + (bh0 + n) * (C * V) + v0 + row * V + (lane % PU) * 8, b + L::s_u + ins * 1024);
+      if (lane < K / 4) dma16(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
+    };
+    // instructions of one chunk per wave: the wait that leaves only the newest chunk's outstanding
+    constexpr int PER = (3 * C * L::RB + C * L::CB) / 1024 / NL + 2;
+    static_assert(2 * PER <= 63, "two chunks' loads fit the wait counter");
+    issue_ka(0);
+    issue_wq(0);
+    if (last > 0) {
+      issue_ka(1);
+      issue_wq(1);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER));
+    } else {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    }
+    bare_barrier();
+    for (int n = 0; n < dm.NT; ++n) {
+      const bool more = n + 2 <= last;
+      if (more) issue_ka(n + 2);   // its buffer was read last before step n - 1's first barrier
+      bare_barrier();
+      if (more) {
+        issue_wq(n + 2);           // its buffer was read last before this barrier
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER));
+      } else {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      }
+      bare_barrier();
+    }
+    return;
   }
 
-  // X tiles: rows [0, C) = w_pseudo h, rows [C, 2C) = qg h; (2C/16) x NTI tiles
-  constexpr int NTX = (2 * C / 16) * NTI;
-  constexpr int XPW = NTX / NW;
-  static_assert(NTX % NW == 0 && XPW >= 1, "output tiles must split evenly over the waves");
-  // tiles of one row block computed together (sharing their A fragments)
-  constexpr int GX = XPW < NTI ? XPW : NTI, GT = TPW < NTI ? TPW : NTI;
-  static_assert(XPW % GX == 0 && NTI % GX == 0 && TPW % GT == 0 && NTI % GT == 0, "tile groups");
-
-  // the chunk operands move global -> registers -> LDS; two register sets
-  // keep the loads of chunk n + 2 in flight while chunk n computes
-  struct Stage {
-    RegStage<T, C, K, NTHR> w, q, k;
-    RegStage<T, C, C, NTHR> a;
-    RegStage<T, C, VT, NTHR> u;
-    RegStage<float, 1, K, NTHR> g;
-  };
-  auto prefetch = [&](Stage& S, int n) {
-    const size_t bhn = (size_t)bh * dm.NT + n;
-    S.w.load(ck.wt + bhn * C * K, K);
-    S.q.load(ck.qg + bhn * C * K, K);
-    S.k.load(ck.kg + bhn * C * K, K);
-    S.a.load(ck.aqk + bhn * C * C, C);
-    S.u.load(ck.u + bhn * C * V + v0, V);
-    S.g.load(ck.gcl + bhn * K, K);
-  };
-  auto commit = [&](const Stage& S, int bsel) {
-    unsigned char* bp = lds + bsel * L::SB;
-    S.w.store(reinterpret_cast<T*>(bp + L::s_w), L::LK);
-    S.q.store(reinterpret_cast<T*>(bp + L::s_q), L::LK);
-    S.k.store(reinterpret_cast<T*>(bp + L::s_kg), L::LK);
-    S.a.store(reinterpret_cast<T*>(bp + L::s_aqk), L::LC);
-    S.u.store(reinterpret_cast<T*>(bp + L::s_u), L::LU);
-    S.g.store(reinterpret_cast<float*>(bp + L::s_gl), K);
-  };
-  // Every prefetch is issued on every path (past the last chunk it re-reads
-  // chunk NT - 1, whose registers are never committed): the wait counter
-  // before a commit then always has the other set's loads behind it, so the
-  // commit waits for its own set only and the two-deep prefetch holds.
-  const int last = dm.NT - 1;
-  Stage s0, s1;
-  prefetch(s0, 0);
-  commit(s0, 0);
-  __syncthreads();
-  prefetch(s0, min(1, last));
-  if constexpr (PD == 2) prefetch(s1, min(2, last));
-
-  const bool chunk_o = (mode & kStateChunkO) != 0;
-  const size_t ors = chunk_o ? (size_t)V : (size_t)dm.H * V;  // o's row stride
-  static_assert(!DO || L::NBUF == 2, "deferred o stores follow the step-start commit");
-  f32x4 po[XPW];
-  float* pog = nullptr;
-  // this wave's o tiles (rows of the qg half) at o's row base og
-  auto store_o = [&](float* og, const f32x4 (&ov)[XPW]) {
+  if (wid < 4) {
+    // ---------------- v_new and the state: h[d][v] with d = 16 (w RB + t) + r16, v = 16 u + 4 g4 + i
+    f32x4 hs[RB][NTI];
 #pragma unroll
-    for (int gi = 0; gi < XPW / GX; ++gi) {
-      const int tile0 = wv_id * XPW + gi * GX, mi = tile0 / NTI, ni0 = tile0 % NTI;
-      if (mi >= C / 16) {
-        const int mo = mi - C / 16;
+    for (int t = 0; t < RB; ++t)
 #pragma unroll
-        for (int u = 0; u < GX; ++u)
+      for (int u = 0; u < NTI; ++u) {
+        const int d = 16 * (w * RB + t) + r16;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int r = 16 * mo + tile_row(i), c = 16 * (ni0 + u) + tile_col();
-            og[(size_t)r * ors + c] = n2n(ov[gi * GX + u][i]);
-          }
-      }
-    }
-  };
-
-  // One chunk step; S holds chunk n + 1 on entry and is refilled with chunk n + 3.
-  // Two stage buffers: chunk n + 1 goes into the other buffer at the start (its
-  // last readers finished before the previous step's final barrier), and only
-  // two barriers are left per step (after v_new, after the new h).
-  auto chunk_step = [&](int n, Stage& S) {
-    const size_t bhn = (size_t)bh * dm.NT + n;
-    use_buf(L::NBUF == 2 ? (n & 1) : 0);
-    if constexpr (L::NBUF == 2) {
-      if (n + 1 < dm.NT) commit(S, (n + 1) & 1);
-      if constexpr (DO) {
-        if (pog) store_o(pog, po);
-        pog = nullptr;
-      }
-      prefetch(S, min(n + 1 + PD, last));
-    }
-      if (save) unstage_rows<T, VT, K, NTHR>(ck.hT + bhn * V * K + (size_t)v0 * K, K, sHt, L::LK);
-
-      // v_new = u - w_pseudo h ; qh = qg h   (GX tiles of one row block share the A reads)
-      f32x4 xo[XPW];
-  #pragma unroll
-      for (int gi = 0; gi < XPW / GX; ++gi) {
-        const int tile0 = wv_id * XPW + gi * GX, mi = tile0 / NTI, ni0 = tile0 % NTI;
-        const bool is_w = mi < C / 16;
-        f32x4 acc[GX];
-  #pragma unroll
-        for (int u = 0; u < GX; ++u) acc[u] = zero4();
-        tile_mma_row<T, false, false, GX>(acc, is_w ? sW : sQ, L::LK, sHt, L::LK,
-                                          16 * (is_w ? mi : mi - C / 16), 16 * ni0, K);
-  #pragma unroll
-        for (int u = 0; u < GX; ++u) {
-          const int ni = ni0 + u;
-          if (is_w) {
-  #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int j = 16 * mi + tile_row(i), vv = 16 * ni + tile_col();
-              acc[u][i] = to_f(sU[j * L::LU + vv]) - acc[u][i];
-            }
-            store_tile_t(sVn, L::LC, 16 * mi, 16 * ni, acc[u]);
-          } else {
-  #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[u][i] *= dm.scale;
-          }
-          xo[gi * GX + u] = acc[u];
+        for (int i = 0; i < 4; ++i) {
+          const float hv = h0 ? h0[((size_t)bh * K + d) * V + v0 + 16 * u + 4 * g4 + i] : 0.f;
+          hs[t][u][i] = (mode & kStateSanitizeH0) ? sanitize(hv) : hv;
         }
+        store4(reinterpret_cast<bf16*>(sH + seq_off<VT>(d, 16 * u + 4 * g4)), hs[t][u]);
+      }
+    __syncthreads();
+    for (int n = 0; n < dm.NT; ++n) {
+      const unsigned char* wq = lds + L::off_wq + (n & 1) * L::WQ;
+      const unsigned char* ka = lds + L::off_ka + (n % 3) * L::KA;
+      // v_new = u - w_pseudo h
+      f32x4 x[NTI];
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) x[u] = zero4();
+#pragma unroll
+      for (int s = 0; s < XK; ++s) {
+        const bf16x8 wf = swz_rowfrag<PK>(wq + L::s_w, 16 * w, s);
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) x[u] = M::mma(seq_colfrag<VT>(sH, u, 32 * s), wf, x[u]);
+      }
+      const int j = 16 * w + r16;
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) {
+        const bf16x4 uv = *reinterpret_cast<const bf16x4*>(wq + L::s_u + j * L::UB + (16 * u + 4 * g4) * 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[u][i] = (float)uv[i] - x[u][i];
+        store4(reinterpret_cast<bf16*>(sVn + seq_off<VT>(j, 16 * u + 4 * g4)), x[u]);
+      }
+      // what does not need v_new: kg's fragments and h e^{gc_last}
+      bf16x8 kt[RB][XC];
+#pragma unroll
+      for (int t = 0; t < RB; ++t) {
+        const int d = 16 * (w * RB + t);
+        const float e = __expf(*reinterpret_cast<const float*>(wq + L::s_gl + (d + r16) * 4));
+#pragma unroll
+        for (int s = 0; s < XC; ++s) kt[t][s] = swz_colfrag<PK>(ka + L::s_kg, d, 32 * s);
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hs[t][u][i] *= e;
       }
       __syncthreads();
-      if (save) unstage_rows<T, VT, C, NTHR>(ck.vnT + bhn * V * C + (size_t)v0 * C, C, sVn, L::LC);
-
-      // o = scale qg h + Aqk v_new   (rows of the qg half)
-      float* og = !o ? nullptr
-                     : chunk_o ? o + (size_t)bhn * C * V + v0
-                               : o + (((size_t)bb * dm.T + (size_t)n * C) * dm.H + h) * V + v0;
-  #pragma unroll
-      for (int gi = 0; gi < XPW / GX; ++gi) {
-        const int tile0 = wv_id * XPW + gi * GX, mi = tile0 / NTI, ni0 = tile0 % NTI;
-        if (mi >= C / 16) {
-          const int mo = mi - C / 16;
-          int kr = 16 * (mo + 1);
-          kr = ((kr + Mma<T>::KS - 1) / Mma<T>::KS) * Mma<T>::KS;
-          if (kr > C) kr = C;
-          f32x4 acc[GX];
-  #pragma unroll
-          for (int u = 0; u < GX; ++u) acc[u] = xo[gi * GX + u];
-          tile_mma_row<T, false, false, GX>(acc, sAqk, L::LC, sVn, L::LC, 16 * mo, 16 * ni0, kr);
-          if constexpr (DO) {
-  #pragma unroll
-            for (int u = 0; u < GX; ++u) po[gi * GX + u] = acc[u];
-          } else if (og) {
-  #pragma unroll
-            for (int u = 0; u < GX; ++u)
-  #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int r = 16 * mo + tile_row(i), c = 16 * (ni0 + u) + tile_col();
-                og[(size_t)r * ors + c] = n2n(acc[u][i]);
-              }
-          }
-        }
-      }
-      if constexpr (DO) pog = og;
-
       // h = sanitize(h e^{gc_last} + kg^T v_new)
-  #pragma unroll
-      for (int gi = 0; gi < TPW / GT; ++gi) {
-        const int tile0 = wv_id * TPW + gi * GT, mi = tile0 / NTI, ni0 = tile0 % NTI;
-        f32x4 acc[GT];
-  #pragma unroll
-        for (int u = 0; u < GT; ++u) {
-          acc[u] = hs[gi * GT + u];
-  #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[u][i] *= __expf(sGl[16 * mi + tile_row(i)]);
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const bf16x8 a = seq_colfrag<VT>(sVn, u, 32 * s);
+#pragma unroll
+          for (int t = 0; t < RB; ++t) hs[t][u] = M::mma(a, kt[t][s], hs[t][u]);
         }
-        tile_mma_row<T, true, false, GT>(acc, sKg, L::LK, sVn, L::LC, 16 * mi, 16 * ni0, C);
-  #pragma unroll
-        for (int u = 0; u < GT; ++u) {
-  #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[u][i] = sanitize(acc[u][i]);
-          hs[gi * GT + u] = acc[u];
+#pragma unroll
+      for (int t = 0; t < RB; ++t)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hs[t][u][i] = sanitize(hs[t][u][i]);
+          store4(reinterpret_cast<bf16*>(sH + seq_off<VT>(16 * (w * RB + t) + r16, 16 * u + 4 * g4)), hs[t][u]);
+        }
+      __syncthreads();
+    }
+    if (h_final) {
+#pragma unroll
+      for (int t = 0; t < RB; ++t)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            h_final[((size_t)bh * K + 16 * (w * RB + t) + r16) * V + v0 + 16 * u + 4 * g4 + i] = hs[t][u][i];
+    }
+  } else {
+    // ---------------- o = scale qg h + Aqk v_new (rows 16 w ...), and the saves
+    const bool save = (mode & kStateSave) != 0;
+    const bool chunk_o = (mode & kStateChunkO) != 0;
+    const size_t ors = chunk_o ? (size_t)V : (size_t)dm.H * V;  // o's row stride
+    __syncthreads();
+    for (int n = 0; n < dm.NT; ++n) {
+      const size_t bhn = bh0 + n;
+      const unsigned char* wq = lds + L::off_wq + (n & 1) * L::WQ;
+      const unsigned char* ka = lds + L::off_ka + (n % 3) * L::KA;
+      f32x4 x[NTI];
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) x[u] = zero4();
+#pragma unroll
+      for (int s = 0; s < XK; ++s) {
+        const bf16x8 qf = swz_rowfrag<PK>(wq + L::s_q, 16 * w, s);
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const bf16x8 a = seq_colfrag<VT>(sH, u, 32 * s);
+          x[u] = M::mma(qf, a, x[u]);
+          if (save && s == w) store_frag_rows(ck.hT + bhn * V * K + (size_t)(v0 + 16 * u) * K + 32 * s, K, a);
         }
       }
-      // sHt was last read by this step's [w; q] h, before the v_new barrier;
-      // with one stage buffer, the staged chunk is still being read here
-      if constexpr (L::NBUF == 1) __syncthreads();
-  #pragma unroll
-      for (int t = 0; t < TPW; ++t) {
-        const int tile = wv_id * TPW + t, mi = tile / NTI, ni = tile % NTI;
-        store_tile_t(sHt, L::LK, 16 * mi, 16 * ni, hs[t]);
+#pragma unroll
+      for (int u = 0; u < NTI; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[u][i] *= dm.scale;
+      bf16x8 af[XC];
+#pragma unroll
+      for (int s = 0; s < XC; ++s) af[s] = swz_rowfrag<8>(ka + L::s_a, 16 * w, s);
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const bf16x8 a = seq_colfrag<VT>(sVn, u, 32 * s);
+          if (32 * s <= 16 * w + 15) x[u] = M::mma(af[s], a, x[u]);  // Aqk is lower triangular
+          if (save && s == w) store_frag_rows(ck.vnT + bhn * V * C + (size_t)(v0 + 16 * u) * C + 32 * s, C, a);
+        }
+      if (o) {
+        float* og = chunk_o ? o + bhn * C * V + v0 : o + (((size_t)bb * dm.T + (size_t)n * C) * dm.H + h) * V + v0;
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) og[(size_t)(16 * w + 4 * g4 + i) * ors + 16 * u + r16] = n2n(x[u][i]);
       }
-    if constexpr (L::NBUF == 1) {
-      if (n + 1 < dm.NT) commit(S, 0);
-      prefetch(S, min(n + 1 + PD, last));
+      __syncthreads();
+    }
+  }
+}
+
+// Sixteen bytes of an fp32 row per lane: row r16, elements k0 + 4 g4 + t; MFMA
+// step t takes element t of every lane (k = k0 + 4 g4 + t), in both operands.
+__device__ __forceinline__ f32x4 f32_col(const float* p, int ld, int i0, int k0) {
+  const int l = lane_id();
+  const float* q = p + (k0 + 4 * (l >> 4)) * ld + i0 + (l & 15);
+  f32x4 v = {q[0], q[ld], q[2 * ld], q[3 * ld]};
+  return v;
+}
+__device__ __forceinline__ f32x4 f32_mma(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) c = Mma<float>::mma(a[t], b[t], c);
+  return c;
+}
+
+// fp32 state loop (two chunks of its operands do not fit the LDS): waves 0-3
+// compute v_new and the state, 4-7 o and the saves, each holding the chunk's w
+// / qg / Aqk row fragments in registers PD chunks ahead; kg passes through LDS
+// (its fragments are columns).  K = 64 at B1 T512 H4: 0.037 -> 0.018 ms; B4
+// T4096 H4 0.270 -> 0.117; K = 128, B4 T1024 H8 0.119 -> 0.065.  From more
+// than one workgroup per CU of 16 columns on, 32 columns are faster (K = 64,
+// 512 workgroups of 16: 0.040, 256 of 32: 0.029; K = 128: 0.155 and 0.116).
+template <int C, int K, int V, int VT, int PD>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn2_fwd_state_f32(
+    Gdn2Dims dm, Gdn2Chunks<float> ck, const float* __restrict__ h0, float* __restrict__ o,
+    float* __restrict__ h_final, int mode) {
+  constexpr int NVT = V / VT, NTI = VT / 16, RB = K / 64, XK = K / 16, XC = C / 16;
+  constexpr int LK = K + 4, LV = VT + 4, KG = C * LK;
+  static_assert(C == 64 && K % 64 == 0, "four row blocks");
+  __shared__ __attribute__((aligned(16))) float lds[2 * KG + K * LV + C * LV];
+  float* sH = lds + 2 * KG;
+  float* sVn = sH + K * LV;
+  int bh, vt;
+  xcd_group_map(blockIdx.x, dm.B * dm.H, NVT, bh, vt);
+  const int h = bh % dm.H, bb = bh / dm.H;
+  const int v0 = vt * VT;
+  const int w = wave_id() & 3, lane = lane_id(), r16 = lane & 15, g4 = lane >> 4;
+  const size_t bh0 = (size_t)bh * dm.NT;
+  const int last = dm.NT - 1;
+
+  if (wave_id() < 4) {
+    f32x4 hs[RB][NTI];
+#pragma unroll
+    for (int t = 0; t < RB; ++t)
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) {
+        const int d = 16 * (w * RB + t) + r16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float hv = h0 ? h0[((size_t)bh * K + d) * V + v0 + 16 * u + 4 * g4 + i] : 0.f;
+          hs[t][u][i] = (mode & kStateSanitizeH0) ? sanitize(hv) : hv;
+        }
+        store4(sH + d * LV + 16 * u + 4 * g4, hs[t][u]);
+      }
+    struct Set {
+      f32x4 w[XK], u[NTI];
+      float gl[RB];
+    };
+    Set S[PD];
+    const int wo = (16 * w + r16) * K + 4 * g4, uo = (16 * w + r16) * V + v0 + 4 * g4;
+    auto load = [&](Set& A, int n) {
+      const float* wr = ck.wt + (bh0 + n) * (C * K);
+      const float* ur = ck.u + (bh0 + n) * (C * V);
+      const float* gr = ck.gcl + (bh0 + n) * K;
+#pragma unroll
+      for (int s = 0; s < XK; ++s) A.w[s] = *reinterpret_cast<const f32x4*>(wr + wo + s * 16);
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) A.u[u] = *reinterpret_cast<const f32x4*>(ur + uo + 16 * u);
+#pragma unroll
+      for (int t = 0; t < RB; ++t) A.gl[t] = gr[16 * (w * RB + t) + r16];
+    };
+#pragma unroll
+    for (int i = 0; i < PD; ++i) load(S[i], min(i, last));
+    __syncthreads();
+    auto step = [&](int n, Set& A) {
+      const float* sKg = lds + (n & 1) * KG;
+      f32x4 x[NTI];
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) x[u] = zero4();
+#pragma unroll
+      for (int s = 0; s < XK; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) x[u] = f32_mma(f32_col(sH, LV, 16 * u, s * 16), A.w[s], x[u]);
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[u][i] = A.u[u][i] - x[u][i];
+        store4(sVn + (16 * w + r16) * LV + 16 * u + 4 * g4, x[u]);
+      }
+      f32x4 kt[RB][XC];
+#pragma unroll
+      for (int t = 0; t < RB; ++t) {
+#pragma unroll
+        for (int s = 0; s < XC; ++s) kt[t][s] = f32_col(sKg, LK, 16 * (w * RB + t), s * 16);
+        const float e = __expf(A.gl[t]);
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hs[t][u][i] *= e;
+      }
+      load(A, min(n + PD, last));
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const f32x4 a = f32_col(sVn, LV, 16 * u, s * 16);
+#pragma unroll
+          for (int t = 0; t < RB; ++t) hs[t][u] = f32_mma(a, kt[t][s], hs[t][u]);
+        }
+#pragma unroll
+      for (int t = 0; t < RB; ++t)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hs[t][u][i] = sanitize(hs[t][u][i]);
+          store4(sH + (16 * (w * RB + t) + r16) * LV + 16 * u + 4 * g4, hs[t][u]);
+        }
+      __syncthreads();
+    };
+    int n = 0;
+    for (; n + PD <= dm.NT; n += PD) {
+#pragma unroll
+      for (int i = 0; i < PD; ++i) step(n + i, S[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < PD; ++i)
+      if (n + i < dm.NT) step(n + i, S[i]);
+    if (h_final) {
+#pragma unroll
+      for (int t = 0; t < RB; ++t)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            h_final[((size_t)bh * K + 16 * (w * RB + t) + r16) * V + v0 + 16 * u + 4 * g4 + i] = hs[t][u][i];
+    }
+  } else {
+    constexpr int PIECES = C * K / 4 / 256, PER_ROW = K / 4;  // 16-byte kg pieces per thread
+    struct Set { f32x4 q[XK], a[XC]; };
+    struct KSet { f32x4 p[PIECES]; };
+    Set S[PD];
+    KSet G[PD];
+    const int tid = threadIdx.x & 255;
+    const int qo = (16 * w + r16) * K + 4 * g4, ao = (16 * w + r16) * C + 4 * g4;
+    auto load = [&](Set& A, int n) {
+      const float* qr = ck.qg + (bh0 + n) * (C * K);
+      const float* ar = ck.aqk + (bh0 + n) * (C * C);
+#pragma unroll
+      for (int s = 0; s < XK; ++s) A.q[s] = *reinterpret_cast<const f32x4*>(qr + qo + s * 16);
+#pragma unroll
+      for (int s = 0; s < XC; ++s) A.a[s] = *reinterpret_cast<const f32x4*>(ar + ao + s * 16);
+    };
+    auto load_kg = [&](KSet& A, int n) {
+      const float* kr = ck.kg + (bh0 + n) * (C * K);
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) A.p[i] = *reinterpret_cast<const f32x4*>(kr + (tid + 256 * i) * 4);
+    };
+    auto commit = [&](const KSet& A, int n) {
+      float* d = lds + (n & 1) * KG;
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) {
+        const int e = tid + 256 * i;
+        *reinterpret_cast<f32x4*>(d + (e / PER_ROW) * LK + (e % PER_ROW) * 4) = A.p[i];
+      }
+    };
+    const bool save = (mode & kStateSave) != 0;
+    const bool chunk_o = (mode & kStateChunkO) != 0;
+    const size_t ors = chunk_o ? (size_t)V : (size_t)dm.H * V;
+    {
+      KSet k0;
+      load_kg(k0, 0);
+#pragma unroll
+      for (int i = 0; i < PD; ++i) {
+        load(S[i], min(i, last));
+        load_kg(G[i], min(i + 1, last));
+      }
+      commit(k0, 0);
     }
     __syncthreads();
-  };
-  // both steps of a pair run on every trip (no path skips the second set's
-  // loads); an odd last chunk runs after the loop
-  int n = 0;
-  if constexpr (PD == 2) {
-    for (; n + 1 < dm.NT; n += 2) {
-      chunk_step(n, s0);
-      chunk_step(n + 1, s1);
-    }
-    if (n < dm.NT) chunk_step(n, s0);
-  } else {
-    for (; n < dm.NT; ++n) chunk_step(n, s0);
-  }
-  if constexpr (DO) {
-    if (pog) store_o(pog, po);
-  }
-  if (h_final) {
+    // B holds chunk n + 1's kg
+    auto step = [&](int n, Set& A, KSet& B) {
+      const size_t bhn = bh0 + n;
+      f32x4 x[NTI];
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int tile = wv_id * TPW + t, mi = tile / NTI, ni = tile % NTI;
+      for (int u = 0; u < NTI; ++u) x[u] = zero4();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * mi + tile_row(i), vv = v0 + 16 * ni + tile_col();
-        h_final[((size_t)bh * K + d) * V + vv] = hs[t][i];
+      for (int s = 0; s < XK; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const f32x4 a = f32_col(sH, LV, 16 * u, s * 16);
+          x[u] = f32_mma(A.q[s], a, x[u]);
+          if (save && (s & 3) == w)
+            *reinterpret_cast<f32x4*>(ck.hT + bhn * V * K + (size_t)(v0 + 16 * u + r16) * K + s * 16 + 4 * g4) = a;
+        }
+#pragma unroll
+      for (int u = 0; u < NTI; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[u][i] *= dm.scale;
+      commit(B, n + 1);   // past the last chunk: a copy nobody reads
+      load_kg(B, min(n + PD + 1, last));
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) {
+          const f32x4 a = f32_col(sVn, LV, 16 * u, s * 16);
+          if (s <= w) x[u] = f32_mma(A.a[s], a, x[u]);   // Aqk is lower triangular
+          if (save && (s & 3) == w)
+            *reinterpret_cast<f32x4*>(ck.vnT + bhn * V * C + (size_t)(v0 + 16 * u + r16) * C + s * 16 + 4 * g4) = a;
+        }
+      if (o) {
+        float* og = chunk_o ? o + bhn * C * V + v0 : o + (((size_t)bb * dm.T + (size_t)n * C) * dm.H + h) * V + v0;
+#pragma unroll
+        for (int u = 0; u < NTI; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) og[(size_t)(16 * w + 4 * g4 + i) * ors + 16 * u + r16] = n2n(x[u][i]);
       }
+      load(A, min(n + PD, last));
+      __syncthreads();
+    };
+    int n = 0;
+    for (; n + PD <= dm.NT; n += PD) {
+#pragma unroll
+      for (int i = 0; i < PD; ++i) step(n + i, S[i], G[i]);
     }
+#pragma unroll
+    for (int i = 0; i < PD; ++i)
+      if (n + i < dm.NT) step(n + i, S[i], G[i]);
   }
 }
 

@@ -183,34 +183,37 @@ static int gdn2_intra_launch(const Gdn2Plan& p, const void* q, const void* k, co
 template <typename T, int K>
 static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const float* h0, float* o,
                              float* h_final, int mode, Launch& L) {
-  constexpr int C = 64, V = K, VT = 32;
+  constexpr int C = 64, V = K;
   hipStream_t st = L.st;
   const int bh = p.dm.B * p.dm.H;
-  if constexpr (sizeof(T) == 2 && K == 128) {
-    // Few (batch, head) pairs (long sequences at batch 1): 16-column V tiles
-    // while they still fit one workgroup per CU (256 CUs).  The chunk step is
-    // shorter and twice the workgroups walk the chunks; every tile re-reads
-    // the chunk's w, q, kg, which its XCD's L2 serves.
-    constexpr int VT16 = 16;
-    if (bh * (V / VT16) <= 256) {
-      return L("gdn2_fwd_state", [&] {
-        hipLaunchKernelGGL((gdn2_fwd_state<T, C, K, V, VT16, 8, 2, true>), dim3((unsigned)(bh * (V / VT16))), dim3(512), 0,
-                           st, p.dm, ck, h0, o, h_final, mode);
-      });
-    }
-  }
-  const unsigned nwg = (unsigned)(bh * (V / VT));
-  // bf16 at K = 128: sixteen waves with one prefetch set (measured 3-5 %
-  // faster than eight waves with two; the same tiles, so the same bits)
-  if constexpr (sizeof(T) == 2 && K == 128) {
-    return L("gdn2_fwd_state", [&] {
-      hipLaunchKernelGGL((gdn2_fwd_state<T, C, K, V, VT, 16, 1>), dim3(nwg), dim3(1024), 0, st, p.dm, ck, h0, o,
-                         h_final, mode);
-    });
-  }
+  // V tiles of 16 columns while they fit one workgroup per CU (256 CUs): the
+  // chunk step is shorter and twice the workgroups walk the chunks; every tile
+  // re-reads the chunk's w, q, kg, which its XCD's L2 serves.  Past that, 32
+  // (B4 T8192 H16 K = 128 without saves: 0.36 ms with 16, 0.25 with 32).
+  const bool narrow = bh * (V / 16) <= 256;
   return L("gdn2_fwd_state", [&] {
-    hipLaunchKernelGGL((gdn2_fwd_state<T, C, K, V, VT>), dim3(nwg), dim3(512), 0, st, p.dm, ck, h0, o,
-                       h_final, mode);
+    if constexpr (sizeof(T) == 2) {
+      // The prefetch wave while the workgroups leave CUs idle, where latency
+      // bounds the step (B1 T32768 H16: 0.62 -> 0.49 ms, B8 T4096 H6 0.170 ->
+      // 0.156); with 256 and more it only adds traffic (B4 T8192 H16: 0.248
+      // without, 0.258 with).
+      if (narrow) {
+        const unsigned nwg = (unsigned)(bh * (V / 16));
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 16, 2>), dim3(nwg), dim3(512 + 64 * (2 + (nwg < 256))), 0, st,
+                           p.dm, ck, h0, o, h_final, mode);
+      } else {
+        const unsigned nwg = (unsigned)(bh * (V / 32));
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg), dim3(512 + 64 * (4 + (nwg < 256))), 0, st,
+                           p.dm, ck, h0, o, h_final, mode);
+      }
+    } else {
+      if (narrow)
+        hipLaunchKernelGGL((gdn2_fwd_state_f32<C, K, V, 16, K == 64 ? 2 : 1>), dim3((unsigned)(bh * (V / 16))),
+                           dim3(512), 0, st, p.dm, ck, h0, o, h_final, mode);
+      else
+        hipLaunchKernelGGL((gdn2_fwd_state_f32<C, K, V, 32, 1>), dim3((unsigned)(bh * (V / 32))), dim3(512), 0, st,
+                           p.dm, ck, h0, o, h_final, mode);
+    }
   });
 }
 
