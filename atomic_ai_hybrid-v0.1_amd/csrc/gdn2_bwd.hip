@@ -1,7 +1,7 @@
 // GDN2 WY chunked backward for gfx950: the B2 -> B1 -> B3 -> B4 -> B5 chain of
 // _gdn2_core_bwd (atomic_ops/kernel_trainable_B6.py:97-181).
 //
-//   gdn2_bwd_dh     one workgroup per (batch, head, V tile), reverse over
+//   gdn2_bwd_dh     (gdn2_bwd_dh_f32 for fp32 operands) one workgroup per (batch, head, V tile), reverse over
 //                   chunks: B2's dv_partial = Aqk^T dO, then B1
 //                   (kernel_bwd_b1_dhu.py:22-39) with the fp32 dh carried in
 //                   MFMA accumulators.  Saves dv_new and the carry entering
@@ -57,13 +57,11 @@ struct DhLds {
   static constexpr int total = off_dvt + VT * LC * (int)sizeof(T);
 };
 
-// Eight waves (two per SIMD): the dh tiles and the dv_new tiles of one V
-// tile split over them by row blocks.  With DD, each step's dv_new tiles stay
-// in registers and are written by the next step between its commit and its
-// prefetch (bf16: 0.350 -> 0.332 ms with 32-column tiles, 0.78 -> 0.77 ms
-// with 16; fp32 at K = 128 has one stage buffer and stores in place).
-template <typename T, typename TD, int C, int K, int V, int VT, bool DD = false>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn2_bwd_dh(
+// fp32 operands (two chunks of them do not fit the LDS at K = 128): eight waves
+// (two per SIMD), the dh tiles and the dv_new tiles of one V tile split over
+// them by row blocks, staging through registers.
+template <typename T, typename TD, int C, int K, int V, int VT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn2_bwd_dh_f32(
     Gdn2Dims dm, Gdn2Chunks<T> ck, Gdn2Grads<T> gr, const TD* __restrict__ dO,
     const float* __restrict__ dh_final, float* __restrict__ dh0) {
   typedef DhLds<T, C, K, V, VT> L;
@@ -168,17 +166,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // commit then always has the other set's loads behind it, so the commit
   // waits for its own set only and the two-deep prefetch holds.
   auto buf_of = [](int n) { return L::NBUF == 2 ? (n & 1) : 0; };
-  static_assert(!DD || L::NBUF == 2, "deferred dv_new stores follow the step-start commit");
-  f32x4 pdv[VPW];
-  T* pdvn = nullptr;
-  auto store_dv = [&](T* dvb) {
-  #pragma unroll
-    for (int gi = 0; gi < ((NTV >= NW || wv_id < NTV) ? VPW / GV : 0); ++gi) {
-      const int tile0 = wv_id * VPW + gi * GV, mj = tile0 / NTI, ni0 = tile0 % NTI;
-  #pragma unroll
-      for (int u = 0; u < GV; ++u) store_tile_n(dvb, V, 16 * mj, 16 * (ni0 + u), pdv[gi * GV + u]);
-    }
-  };
   Stage s0, s1;
   prefetch(s0, dm.NT - 1);
   commit(s0, buf_of(dm.NT - 1));
@@ -195,10 +182,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     use_buf(buf_of(n));
     if constexpr (L::NBUF == 2) {
       if (n > 0) commit(S, buf_of(n - 1));
-      if constexpr (DD) {
-        if (pdvn) store_dv(pdvn);
-        pdvn = nullptr;
-      }
       prefetch(S, max(n - 3, 0));
     }
       // dh_next of chunk n = the carry entering this step
@@ -220,14 +203,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const int ni = ni0 + u;
   #pragma unroll
           for (int i = 0; i < 4; ++i) acc[u][i] = sanitize(acc[u][i]);
-          if constexpr (DD) pdv[gi * GV + u] = acc[u];
-          else store_tile_n(gr.dvn + bhn * C * V + v0, V, 16 * mj, 16 * ni, acc[u]);
+          store_tile_n(gr.dvn + bhn * C * V + v0, V, 16 * mj, 16 * ni, acc[u]);
   #pragma unroll
           for (int i = 0; i < 4; ++i) acc[u][i] = -acc[u][i];
           store_tile_t(sDvT, L::LC, 16 * mj, 16 * ni, acc[u]);
         }
       }
-      if constexpr (DD) pdvn = gr.dvn + bhn * C * V + v0;
       __syncthreads();
 
       // dh = sanitize(qg^T (scale dO) + dh e^{gc_last} - w_pseudo^T dv_new)   (b1:26-37)
@@ -272,9 +253,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     chunk_step(n - 1, s1);
   }
   if (n == 0) chunk_step(0, s0);
-  if constexpr (DD) {
-    if (pdvn) store_dv(pdvn);
-  }
   if (dh0) {
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
@@ -288,6 +266,234 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+template <int C, int K, int VT>
+struct DhSeqLds {
+  static constexpr int RB = K * 2, CB = C * 2, UB = VT * 2;
+  static constexpr int s_w = 0, s_q = C * RB, s_kg = 2 * C * RB, s_a = 3 * C * RB, s_gl = s_a + C * CB;
+  static constexpr int ST = s_gl + K * 4;          // loader waves' part, two of these
+  static constexpr int s_do = 0, s_dos = C * UB;   // dO and scale dO as bf16, two of these
+  static constexpr int DO = 2 * C * UB;
+  static constexpr int off_st = 0, off_do = 2 * ST, off_dh = off_do + 2 * DO;
+  static constexpr int off_dv = off_dh + K * UB;
+  static constexpr int off_pf = off_dv + C * UB;
+  static constexpr int total = off_pf + 256;
+  static_assert(total <= 160 * 1024, "one workgroup per CU");
+};
+
+// bf16 dh loop of one (batch, head, VT columns), one workgroup per CU: waves
+// 0-7 compute (a dv_new tile and one 16-row block of dh each), the next NL load
+// the chunks (gdn2_seq.hpp), two bring dO in (it may be fp32 and row-strided, so
+// it passes through registers, to bf16) and one touches the lines of the chunk
+// four steps on.  As in the forward loop everything is computed transposed,
+// and every product that does not need dv_new runs before the barrier that
+// waits for it.  Bound by the step's chain (1.2 us a chunk at 16 columns, 1.45
+// at 32 with the operands in L2; the former kernel, which staged through
+// registers, 1.5 and 2.6) and by HBM at 256 workgroups.
+// B4 T8192 H16, fp32 dO: 0.340 -> 0.297 ms; B8 T4096 H6 0.159 -> 0.127 ms; B1
+// T32768 H16 0.761 -> 0.607 ms (0.769 without the prefetch wave); K = 64, B2
+// T4096 H16 0.081 -> 0.060 ms.
+template <typename TD, int C, int K, int V, int VT, int NL>
+__global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
+    Gdn2Dims dm, Gdn2Chunks<bf16> ck, Gdn2Grads<bf16> gr, const TD* __restrict__ dO,
+    const float* __restrict__ dh_final, float* __restrict__ dh0) {
+  typedef DhSeqLds<C, K, VT> L;
+  typedef Mma<bf16> M;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[L::total];
+  constexpr int NVT = V / VT, NTI = VT / 16, XK = K / 32, XC = C / 32;
+  constexpr int PK = K / 8;
+  constexpr int DT = K / 16;               // d blocks of the state
+  constexpr int NV = 4 * NTI;              // dv_new tiles, one a wave
+  static_assert(C == 64 && NV <= 8 && DT <= 8, "one tile a wave");
+  int bh, vt;
+  xcd_group_map(blockIdx.x, dm.B * dm.H, NVT, bh, vt);
+  const int h = bh % dm.H, bb = bh / dm.H;
+  const int v0 = vt * VT;
+  const int wid = wave_id(), lane = lane_id(), r16 = lane & 15, g4 = lane >> 4;
+  const size_t bh0 = (size_t)bh * dm.NT;
+  const int last = dm.NT - 1;
+  unsigned char* sDh = lds + L::off_dh;
+  unsigned char* sDv = lds + L::off_dv;
+  // chunk of step i: NT - 1 - i; its buffers: i & 1
+  if (wid == 8 + NL + 2) {
+    // ---------------- L2 prefetch, four chunks ahead; the V tiles of a head share an XCD and split its lines
+    auto touch = [&](const void* p, int bytes) { touch_lines(p, bytes, NVT, vt, lds + L::off_pf); };
+    auto pf = [&](int i) {
+      if (i > last) return;
+      const int n = last - i;
+      touch(ck.wt + (bh0 + n) * (C * K), C * K * 2);
+      touch(ck.qg + (bh0 + n) * (C * K), C * K * 2);
+      touch(ck.kg + (bh0 + n) * (C * K), C * K * 2);
+      touch(ck.aqk + (bh0 + n) * (C * C), C * C * 2);
+    };
+    pf(2); pf(3);
+    bare_barrier();
+    for (int i = 0; i < dm.NT; ++i) { pf(i + 4); bare_barrier(); bare_barrier(); }
+    return;
+  }
+  if (wid >= 8 && wid < 8 + NL) {
+    // ---------------- loader waves
+    const int lw = wid - 8;
+    auto issue = [&](int i) {
+      const int n = last - i;
+      unsigned char* b = lds + L::off_st + (i & 1) * L::ST;
+      dma_rows<K, NL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
+      dma_rows<K, NL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
+      dma_rows<K, NL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
+      dma_rows<C, NL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
+      if (lane < K / 4) dma16(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
+    };
+    // instructions of one chunk per wave: the wait that leaves only the newest chunk's outstanding
+    constexpr int PER = (3 * C * L::RB + C * L::CB) / 1024 / NL + 1;
+    static_assert(2 * PER <= 63, "two chunks' loads fit the wait counter");
+    issue(0);
+    if (last > 0) { issue(1); __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER)); }
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    bare_barrier();
+    for (int i = 0; i < dm.NT; ++i) {
+      bare_barrier();
+      if (i + 2 <= last) { issue(i + 2); __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER)); }
+      else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      bare_barrier();
+    }
+    return;
+  }
+  if (wid >= 8 + NL) {
+    // ---------------- dO: 32 rows a wave, to bf16 (and scaled)
+    const int dw = wid - 8 - NL;
+    constexpr int PPR = VT / 8;                  // 8-element pieces a row
+    constexpr int PT = 32 * PPR / 64;            // pieces a lane
+    static_assert(PT >= 1, "whole waves of pieces");
+    struct Set { Raw8<TD> r[PT]; };
+    const TD* base = dO + (size_t)bb * dm.T * dm.rdo + (size_t)h * V + v0;
+    auto load = [&](Set& S, int i) {
+      const int n = last - min(i, last);
+#pragma unroll
+      for (int p = 0; p < PT; ++p) {
+        const int e = lane + 64 * p, row = 32 * dw + e / PPR;
+        S.r[p].load(base + ((size_t)n * C + row) * dm.rdo + (e % PPR) * 8);
+      }
+    };
+    auto put = [&](const Set& S, int i) {
+      unsigned char* b = lds + L::off_do + (i & 1) * L::DO;
+#pragma unroll
+      for (int p = 0; p < PT; ++p) {
+        const int e = lane + 64 * p, row = 32 * dw + e / PPR, col = (e % PPR) * 8;
+        float x[8], y[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { x[j] = S.r[p][j]; y[j] = x[j] * dm.scale; }
+        store8(reinterpret_cast<bf16*>(b + L::s_do + seq_off<VT>(row, col)), x);
+        store8(reinterpret_cast<bf16*>(b + L::s_dos + seq_off<VT>(row, col)), y);
+      }
+    };
+    Set s0, s1;
+    load(s0, 0);
+    load(s1, 1);
+    put(s0, 0);
+    load(s0, 2);
+    __syncthreads();
+    // step i: the buffer of step i + 1 was read last in step i - 1
+    auto step = [&](int i, Set& S) {
+      put(S, i + 1);
+      load(S, i + 3);
+      __syncthreads();
+      __syncthreads();
+    };
+    int i = 0;
+    for (; i + 2 <= dm.NT; i += 2) { step(i, s1); step(i + 1, s0); }
+    if (i < dm.NT) step(i, s1);
+    return;
+  }
+
+  const int w = wid;
+  const bool has_d = w < DT, has_v = w < NV;
+  const int jb = w & 3, vu = w >> 2;     // this wave's dv_new tile: rows 16 jb, columns 16 vu
+  f32x4 hs[NTI];
+  if (has_d) {
+#pragma unroll
+    for (int u = 0; u < NTI; ++u) {
+      const int d = 16 * w + r16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        hs[u][i] = dh_final ? sanitize(dh_final[((size_t)bh * K + d) * V + v0 + 16 * u + 4 * g4 + i]) : 0.f;
+      store4(reinterpret_cast<bf16*>(sDh + seq_off<VT>(d, 16 * u + 4 * g4)), hs[u]);
+    }
+  }
+  __syncthreads();
+  for (int i = 0; i < dm.NT; ++i) {
+    const int n = last - i;
+    const size_t bhn = bh0 + n;
+    const unsigned char* st = lds + L::off_st + (i & 1) * L::ST;
+    const unsigned char* sd = lds + L::off_do + (i & 1) * L::DO;
+    if (has_v) {
+      // dv_new = sanitize(Aqk^T dO + kg dh)
+      f32x4 x = zero4();
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+        if (32 * s + 31 >= 16 * jb)   // Aqk is lower triangular
+          x = M::mma(seq_colfrag<VT>(sd + L::s_do, vu, 32 * s), swz_colfrag<8>(st + L::s_a, 16 * jb, 32 * s), x);
+      const int j = 16 * jb + r16;
+#pragma unroll
+      for (int s = 0; s < XK; ++s) {
+        const bf16x8 kf = swz_rowfrag<PK>(st + L::s_kg, 16 * jb, s);
+        const bf16x8 a = seq_colfrag<VT>(sDh, vu, 32 * s);
+        x = M::mma(a, kf, x);
+        if (s == jb)   // dh_next of chunk n = the carry entering this step
+          store_frag_rows(gr.dhT + bhn * V * K + (size_t)(v0 + 16 * vu) * K + 32 * s, K, a);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = -sanitize(x[q]);
+      store4(reinterpret_cast<bf16*>(sDv + seq_off<VT>(j, 16 * vu + 4 * g4)), x);
+    }
+    bf16x8 wf[XC];
+    if (has_d) {
+      // dh = sanitize(qg^T (scale dO) + dh e^{gc_last} - w_pseudo^T dv_new): all but the last term
+      const float e = __expf(*reinterpret_cast<const float*>(st + L::s_gl + (16 * w + r16) * 4));
+#pragma unroll
+      for (int u = 0; u < NTI; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) hs[u][q] *= e;
+#pragma unroll
+      for (int s = 0; s < XC; ++s) {
+        const bf16x8 qf = swz_colfrag<PK>(st + L::s_q, 16 * w, 32 * s);
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) hs[u] = M::mma(seq_colfrag<VT>(sd + L::s_dos, u, 32 * s), qf, hs[u]);
+        wf[s] = swz_colfrag<PK>(st + L::s_w, 16 * w, 32 * s);
+      }
+    }
+    __syncthreads();
+    if (has_d) {
+#pragma unroll
+      for (int s = 0; s < XC; ++s)
+#pragma unroll
+        for (int u = 0; u < NTI; ++u) hs[u] = M::mma(seq_colfrag<VT>(sDv, u, 32 * s), wf[s], hs[u]);
+#pragma unroll
+      for (int u = 0; u < NTI; ++u) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) hs[u][q] = sanitize(hs[u][q]);
+        store4(reinterpret_cast<bf16*>(sDh + seq_off<VT>(16 * w + r16, 16 * u + 4 * g4)), hs[u]);
+      }
+    }
+    // dv_new rows out (LDS holds them negated): 16-byte pieces over the eight waves
+    {
+      constexpr int PPR = VT / 8;
+      const int e = threadIdx.x;
+      if (e < C * PPR) {
+        const int row = e / PPR, col = (e % PPR) * 8;
+        u32x4 p = *reinterpret_cast<const u32x4*>(sDv + seq_off<VT>(row, col));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) p[q] ^= 0x80008000u;
+        *reinterpret_cast<u32x4*>(gr.dvn + bhn * C * V + (size_t)row * V + v0 + col) = p;
+      }
+    }
+    __syncthreads();
+  }
+  if (dh0 && has_d) {
+#pragma unroll
+    for (int u = 0; u < NTI; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dh0[((size_t)bh * K + 16 * w + r16) * V + v0 + 16 * u + 4 * g4 + i] = hs[u][i];
+  }
+}
 // ------------------------------------------------------------------ B2/B3 state terms
 // One workgroup per (batch, head, chunk).  dO, dv_new and v_new stay in LDS;
 // h_pre and dh_next ([V][K] per chunk) pass through in quarters of VQ whole
