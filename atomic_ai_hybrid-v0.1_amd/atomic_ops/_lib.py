@@ -219,6 +219,9 @@ _SIGS = {
     "atomic_norm_gate_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(NormGateArgs)]),
     "atomic_norm_gate_fwd": (ctypes.c_int, [ctypes.POINTER(NormGateArgs)] + [_P] * 4 + [_P]),
     "atomic_norm_gate_bwd": (ctypes.c_int, [ctypes.POINTER(NormGateArgs)] + [_P] * 7 + [_P, ctypes.c_size_t, _P]),
+    "atomic_norm_gate_fwd_rows": (ctypes.c_int, [ctypes.POINTER(NormGateArgs), _P, _P, ctypes.c_int64, _P, _P, _P]),
+    "atomic_norm_gate_bwd_rows": (ctypes.c_int, [ctypes.POINTER(NormGateArgs), _P, _P, ctypes.c_int64] + [_P] * 5
+                                  + [_P, ctypes.c_size_t, _P]),
     "atomic_gdn2_prologue_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(PrologueArgs)]),
     "atomic_gdn2_prologue_fwd": (ctypes.c_int, [ctypes.POINTER(PrologueArgs)] + [_P] * 15 + [_P]),
     "atomic_gdn2_prologue_bwd": (ctypes.c_int, [ctypes.POINTER(PrologueArgs)] + [_P] * 24 + [_P, ctypes.c_size_t, _P]),

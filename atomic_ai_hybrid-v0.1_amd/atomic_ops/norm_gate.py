@@ -42,7 +42,13 @@ def _prep(x, gate, weight):
     if gate.dtype != torch.bfloat16 or gate.numel() != x.numel():
         raise TypeError("gate must be bfloat16 with x's number of elements")
     rows = x.numel() // d
-    return x.contiguous().view(rows, d), gate.contiguous().view(rows, d), weight.contiguous(), rows, d
+    # rows of a wider tensor are read in place; the rows have to be d wide
+    stride = 0
+    if gate.dim() >= 3 and gate.numel() == gate.shape[0] * gate.shape[1] * d:
+        gate, stride = _lib.row_view(gate)
+    if not stride:
+        gate = gate.contiguous()
+    return x.contiguous().view(rows, d), gate, stride or d, weight.contiguous(), rows, d
 
 
 def make_args(rows, d, variant, eps):
@@ -52,21 +58,21 @@ def make_args(rows, d, variant, eps):
 def forward(x, gate, weight, variant, eps=1e-6, *, timer=None):
     """``out`` [rows, d] bf16 (the shape of gate)."""
     shape = gate.shape
-    x2, g2, w, rows, d = _prep(x, gate, weight)
+    x2, g2, gs, w, rows, d = _prep(x, gate, weight)
     lib = _lib.load()
     args = make_args(rows, d, variant, eps)
     if timer is not None:
         args.profile = timer.arm()
     out = torch.empty(rows, d, dtype=torch.bfloat16, device=x.device)
-    rc = lib.atomic_norm_gate_fwd(ctypes.byref(args), _ptr(x2), _ptr(g2), _ptr(w), _ptr(out),
-                                  _stream(x.device))
-    _lib.check(rc, "atomic_norm_gate_fwd")
+    rc = lib.atomic_norm_gate_fwd_rows(ctypes.byref(args), _ptr(x2), _ptr(g2), gs, _ptr(w), _ptr(out),
+                                       _stream(x.device))
+    _lib.check(rc, "atomic_norm_gate_fwd_rows")
     return out.view(shape)
 
 
 def backward(x, gate, weight, dout, variant, eps=1e-6, *, workspace=None, timer=None):
     """``(dx, dgate, dweight)`` in x's, gate's and weight's shapes and dtypes."""
-    x2, g2, w, rows, d = _prep(x, gate, weight)
+    x2, g2, gs, w, rows, d = _prep(x, gate, weight)
     lib = _lib.load()
     args = make_args(rows, d, variant, eps)
     if timer is not None:
@@ -80,10 +86,10 @@ def backward(x, gate, weight, dout, variant, eps=1e-6, *, workspace=None, timer=
     dx = torch.empty(rows, d, dtype=torch.float32, device=x.device)
     dg = torch.empty(rows, d, dtype=torch.bfloat16, device=x.device)
     dw = torch.empty(d, dtype=torch.float32, device=x.device)
-    rc = lib.atomic_norm_gate_bwd(ctypes.byref(args), _ptr(x2), _ptr(g2), _ptr(w), _ptr(do2), _ptr(dx),
-                                  _ptr(dg), _ptr(dw), _ptr(workspace), ctypes.c_size_t(workspace.numel()),
-                                  _stream(x.device))
-    _lib.check(rc, "atomic_norm_gate_bwd")
+    rc = lib.atomic_norm_gate_bwd_rows(ctypes.byref(args), _ptr(x2), _ptr(g2), gs, _ptr(w), _ptr(do2), _ptr(dx),
+                                       _ptr(dg), _ptr(dw), _ptr(workspace), ctypes.c_size_t(workspace.numel()),
+                                       _stream(x.device))
+    _lib.check(rc, "atomic_norm_gate_bwd_rows")
     return dx.view(x.shape), dg.view(gate.shape), dw
 
 

@@ -580,6 +580,17 @@ int atomic_norm_gate_bwd(const atomic_norm_gate_args* a, const float* x, const v
                          const float* weight, const void* dout, float* dx, void* dgate,
                          float* dweight, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same two with gate's row stride in elements: gate may be a slice of a
+ * wider [rows, F] tensor (the second half of a Mamba2 block's in_proj output,
+ * reference model.py:405-406) and is read in place.  At least dim, a multiple
+ * of 8, gate 16-byte aligned (ATOMIC_ERR_SHAPE otherwise); dgate is dense. */
+int atomic_norm_gate_fwd_rows(const atomic_norm_gate_args* a, const float* x, const void* gate,
+                              int64_t gate_stride, const float* weight, void* out, void* stream);
+int atomic_norm_gate_bwd_rows(const atomic_norm_gate_args* a, const float* x, const void* gate,
+                              int64_t gate_stride, const float* weight, const void* dout, float* dx,
+                              void* dgate, float* dweight, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 /* ------------------------------------------- GDN2 prologue (upstream) */
 
 /* The GDN2 block's prologue, fused: from the projection outputs to the

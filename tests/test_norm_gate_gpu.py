@@ -76,6 +76,29 @@ def test_autograd_wrapper_and_shapes():
     assert rel_err(wc.grad, dw_ref) < TOL_BF16
 
 
+@pytest.mark.parametrize("variant,ovar", VARIANTS)
+@pytest.mark.parametrize("B,T,d,width,off", [
+    (1, 5, 512, 1024, 512),     # one batch row, fewer rows than a workgroup's four
+    (2, 33, 1536, 3072, 1536),  # the second half of an in_proj output
+    (1, 9, 4096, 4104, 8),      # a workgroup per row; the narrowest slice that starts past column 0
+    (2, 6, 512, 1028, 512),     # rows that are not whole 16-byte pieces: copied
+    (2, 6, 512, 1024, 4),       # a slice that does not start on 16 bytes: copied
+])
+def test_gate_read_in_place_matches_a_dense_gate(variant, ovar, B, T, d, width, off):
+    """A gate that is a slice of a wider tensor gives the dense gate's results bit for bit."""
+    banner(f"norm_gate strided gate {ovar} B{B} T{T} d={d} width={width} off={off}")
+    g = torch.Generator().manual_seed(d + off)
+    x = torch.randn(B, T, d, generator=g).cuda()
+    wide = torch.randn(B, T, width, generator=g).to(torch.bfloat16).cuda()
+    gate = wide[..., off:off + d]
+    w = (1.0 + 0.1 * torch.randn(d, generator=g)).cuda()
+    dout = torch.randn(B, T, d, generator=g).to(torch.bfloat16).cuda()
+    got = (NG.forward(x, gate, w, variant), *NG.backward(x, gate, w, dout, variant))
+    dense = (NG.forward(x, gate.contiguous(), w, variant), *NG.backward(x, gate.contiguous(), w, dout, variant))
+    for a, b in zip(got, dense):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
 def test_unsupported_dimension_is_rejected_before_launch():
     banner("norm_gate shape error")
     x = torch.zeros(4, 640, device="cuda")
