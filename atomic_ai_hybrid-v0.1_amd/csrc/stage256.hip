@@ -656,11 +656,21 @@ __global__ __launch_bounds__(256) void m256_state_pass_k(Mamba2Dims d, const flo
   const size_t bh = e / ((size_t)P * N);
   const int bb = (int)(bh / d.H), h = (int)(bh % d.H);
   float st = state0 ? sanitize(state0[e]) : 0.f;
-  for (int n = 0; n < d.NT; ++n) {
-    const size_t bhn = bh * d.NT + n;
-    pre[((((size_t)bb * d.NT + n) * d.H + h) * P + p) * N + s] = st;
-    const float cl = cum[(bhn * d.C + d.C - 1) * P + p];
-    st = sanitize(st * __expf(fminf(fmaxf(cl, -kClipDecay), 0.f)) + state_end[(bhn * P + p) * N + s]);
+  constexpr int U = 8;  // chunks' values in flight
+  for (int n0 = 0; n0 < d.NT; n0 += U) {
+    float se[U], cl[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t bhn = bh * d.NT + min(n0 + u, d.NT - 1);
+      se[u] = state_end[(bhn * P + p) * N + s];
+      cl[u] = cum[(bhn * d.C + d.C - 1) * P + p];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (n0 + u >= d.NT) break;
+      pre[((((size_t)bb * d.NT + n0 + u) * d.H + h) * P + p) * N + s] = st;
+      st = sanitize(st * __expf(fminf(fmaxf(cl[u], -kClipDecay), 0.f)) + se[u]);
+    }
   }
   state_final[e] = st;
 }

@@ -19,8 +19,15 @@ struct StageIn {
   const void* p;
   int bf;  // 1: bf16, 0: fp32
 };
+// One dword load whatever the type (a bf16 element is one half of the aligned
+// dword that holds it), and selects: a branch on the type around each load
+// kept a loop's loads from being in flight together (eight of them in turn
+// were most of a GEMM tile's 28 us).
 __device__ __forceinline__ float ld(const StageIn& a, size_t i) {
-  return a.bf ? to_f(reinterpret_cast<const bf16*>(a.p)[i]) : reinterpret_cast<const float*>(a.p)[i];
+  const uintptr_t q = reinterpret_cast<uintptr_t>(a.p) + (i << (a.bf ? 1 : 2));
+  const uint32_t w = *reinterpret_cast<const uint32_t*>(q & ~(uintptr_t)3);
+  const uint32_t h = (q & 2) ? w & 0xffff0000u : w << 16;
+  return __uint_as_float(a.bf ? h : w);
 }
 
 // GDN2 (dims with C = 256, NT = T / 256; K = V in {64, 128}); dtype is the

@@ -63,67 +63,95 @@ struct GemmOp {
   int accum, mask, post;
 };
 
-constexpr int GT = 64, GK = 16;
+constexpr int GT = 64, GK = 32;
 
+// 64 x 64 tiles, four waves of 32 x 32 on 16x16x4 fp32 MFMA; k in steps of 32
+// through LDS, the next step's elements in registers while this one computes.
+// LDS rows [m][k] of GK + 4 floats put a fragment's 64 elements on distinct
+// banks.  k ascends through the MFMAs: the sums are those of a serial fma chain
+// (mamba2's dA cancels to 1e-4 of its terms and shows another order).  At 64 x
+// 64 x 64 per item and 512 items the calls are latency: the former vector-ALU
+// tile, with a branch per load, took 28 us a launch, this one 15.
 __global__ __launch_bounds__(256) void sb_gemm_k(GemmOp g) {
-  __shared__ __attribute__((aligned(16))) float sA[GK][GT + 4];
-  __shared__ __attribute__((aligned(16))) float sB[GK][GT + 4];
+  constexpr int LK = GK + 4, NE = GT * GK / 256;
+  __shared__ __attribute__((aligned(16))) float sA[GT][LK];
+  __shared__ __attribute__((aligned(16))) float sB[GT][LK];
   const int z = blockIdx.z;
   const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-  const int t = threadIdx.x, tx = t % 16, ty = t / 16;
+  const int t = threadIdx.x, lane = lane_id(), r16 = lane & 15, g4 = lane >> 4;
+  const int wm = 32 * (wave_id() >> 1), wn = 32 * (wave_id() & 1);
   const size_t oa = bat_off(g.sa, z, g.Z1, g.Z0), ob = bat_off(g.sb, z, g.Z1, g.Z0);
-  float acc[4][4];
+  f32x4 acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int j = 0; j < 2; ++j) acc[i][j] = zero4();
+  float ra[NE], rb[NE];
+  // element it of this thread: row (m or n) and k of the tile, the memory's fast index fastest
+  auto at = [&](int it, bool kfast, int& r, int& k) {
+    const int e = t + 256 * it;
+    r = kfast ? e / GK : e % GT;
+    k = kfast ? e % GK : e / GT;
+  };
+  // past the edge: the last row / k again, zeroed (every load in bounds and unconditional)
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int it = 0; it < NE; ++it) {
+      int r, kk;
+      at(it, !g.ta, r, kk);
+      const int m = min(m0 + r, g.M - 1), k = min(k0 + kk, g.K - 1);
+      ra[it] = ld(g.A, oa + (g.ta ? (size_t)k * g.lda + m : (size_t)m * g.lda + k));
+      if (m0 + r >= g.M || k0 + kk >= g.K) ra[it] = 0.f;
+      at(it, g.tb, r, kk);
+      const int n = min(n0 + r, g.N - 1), kq = min(k0 + kk, g.K - 1);
+      rb[it] = ld(g.B, ob + (g.tb ? (size_t)n * g.ldb + kq : (size_t)kq * g.ldb + n));
+      if (n0 + r >= g.N || k0 + kk >= g.K) rb[it] = 0.f;
+    }
+  };
+  load(0);
   for (int k0 = 0; k0 < g.K; k0 += GK) {
+    __syncthreads();  // the previous step's fragments are read
 #pragma unroll
-    for (int it = 0; it < GT * GK / 256; ++it) {
-      const int e = t + 256 * it;
-      const int mm = g.ta ? e % GT : e / GK, kk = g.ta ? e / GT : e % GK;
-      const int m = m0 + mm, k = k0 + kk;
-      sA[kk][mm] = (m < g.M && k < g.K)
-                       ? ld(g.A, oa + (g.ta ? (size_t)k * g.lda + m : (size_t)m * g.lda + k))
-                       : 0.f;
-      const int nn = g.tb ? e / GK : e % GT, kb = g.tb ? e % GK : e / GT;
-      const int n = n0 + nn, kq = k0 + kb;
-      sB[kb][nn] = (n < g.N && kq < g.K)
-                       ? ld(g.B, ob + (g.tb ? (size_t)n * g.ldb + kq : (size_t)kq * g.ldb + n))
-                       : 0.f;
+    for (int it = 0; it < NE; ++it) {
+      int r, kk;
+      at(it, !g.ta, r, kk);
+      sA[r][kk] = ra[it];
+      at(it, g.tb, r, kk);
+      sB[r][kk] = rb[it];
     }
     __syncthreads();
+    if (k0 + GK < g.K) load(k0 + GK);
 #pragma unroll
-    for (int kk = 0; kk < GK; ++kk) {
-      float a[4], b[4];
+    for (int ks = 0; ks < GK; ks += Mma<float>::KS) {
+      float a[2], b[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = sA[kk][ty + 16 * i];
-      const float4 bv = *reinterpret_cast<const float4*>(&sB[kk][4 * tx]);
-      b[0] = bv.x; b[1] = bv.y; b[2] = bv.z; b[3] = bv.w;
+      for (int i = 0; i < 2; ++i) {
+        a[i] = sA[wm + 16 * i + r16][ks + g4];
+        b[i] = sB[wn + 16 * i + r16][ks + g4];
+      }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < 2; ++j) acc[i][j] = Mma<float>::mma(a[i], b[j], acc[i][j]);
     }
-    __syncthreads();
   }
   const size_t oc = bat_off(g.sc, z, g.Z1, g.Z0);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty + 16 * i;
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + 4 * tx + j;
-      if (m >= g.M || n >= g.N) continue;
-      const size_t o = oc + (size_t)m * g.ldc + n;
-      float v = g.alpha * acc[i][j];
-      if (g.accum) v = g.C[o] + v;
-      if ((g.mask == 1 && n > m) || (g.mask == 2 && n >= m)) v = 0.f;
-      if (g.post == 1) v = n2n_acc(v);
-      else if (g.post == 2) v = sanitize(v);
-      g.C[o] = v;
-    }
-  }
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int m = m0 + wm + 16 * i + 4 * g4 + q, n = n0 + wn + 16 * j + r16;
+        if (m >= g.M || n >= g.N) continue;
+        const size_t o = oc + (size_t)m * g.ldc + n;
+        float v = g.alpha * acc[i][j][q];
+        if (g.accum) v = g.C[o] + v;
+        if ((g.mask == 1 && n > m) || (g.mask == 2 && n >= m)) v = 0.f;
+        if (g.post == 1) v = n2n_acc(v);
+        else if (g.post == 2) v = sanitize(v);
+        g.C[o] = v;
+      }
 }
 
 int gemm(const GemmOp& g, int batch, const char* name, Launch& L) {
@@ -650,10 +678,6 @@ __global__ __launch_bounds__(256) void m2b_headsum_k(Mamba2Dims d, const float* 
   dC[e] = sc;
 }
 
-__global__ __launch_bounds__(256) void fill0_k(float* __restrict__ p, size_t n) {
-  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) p[e] = 0.f;
-}
-
 // ------------------------------------------------------------------ Mamba2 MB1 + MB3, MB4
 // The reference's trainable Mamba2 backward (kernel_mamba2_trainable_B6.py:
 // 83-131): mamba2_bwd_scan (kernel_mamba2_bwd_b1_state.py:132-254) re-runs
@@ -725,13 +749,23 @@ __global__ __launch_bounds__(256) void m2s_fwd_pass_k(Mamba2Dims d, const float*
   const size_t bh = e / ((size_t)d.P * d.N);
   const int h = (int)(bh % d.H), b = (int)(bh / d.H);
   float st = state0 ? sanitize(state0[e]) : 0.f;
-  for (int n = 0; n < d.NT; ++n) {
-    const size_t o = ((((size_t)b * d.NT + n) * d.H + h) * d.P + p) * d.N + s;
-    const float se = sprev[o];
-    sprev[o] = st;
-    const float cl = cum[((bh * d.NT + n) * d.C + d.C - 1) * d.P + p];
-    const float dce = __expf(fminf(fmaxf(cl, -kClipDecay), 0.f));                                  // :144
-    st = sanitize(st * dce + sanitize(se));                                                        // :136-137,145-146
+  // U chunks' values in flight (each is read before any of the U is replaced)
+  constexpr int U = 8;
+  for (int n0 = 0; n0 < d.NT; n0 += U) {
+    float se[U], cl[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = min(n0 + u, d.NT - 1);
+      se[u] = sprev[((((size_t)b * d.NT + n) * d.H + h) * d.P + p) * d.N + s];
+      cl[u] = cum[((bh * d.NT + n) * d.C + d.C - 1) * d.P + p];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (n0 + u >= d.NT) break;
+      sprev[((((size_t)b * d.NT + n0 + u) * d.H + h) * d.P + p) * d.N + s] = st;
+      const float dce = __expf(fminf(fmaxf(cl[u], -kClipDecay), 0.f));                             // :144
+      st = sanitize(st * dce + sanitize(se[u]));                                                   // :136-137,145-146
+    }
   }
 }
 
@@ -819,14 +853,23 @@ __global__ __launch_bounds__(256) void m2s_bwd_pass_k(Mamba2Dims d, const float*
   const int s = (int)(e % d.N), p = (int)((e / d.N) % d.P);
   const size_t bh = e / ((size_t)d.P * d.N);
   float car = dsf ? dsf[e] : 0.f;
-  for (int n = d.NT - 1; n >= 0; --n) {
-    const size_t z = bh * d.NT + n;
-    const size_t o = (z * d.P + p) * d.N + s;
-    const float acc = dse[o];
-    const float c = sanitize(car);
-    dse[o] = c;
-    const float dce = __expf(fminf(fmaxf(cum[(z * d.C + d.C - 1) * d.P + p], -kClipDecay), 0.f));
-    car = sanitize(c * dce + acc);
+  // U chunks' values in flight (each is read before any of the U is replaced)
+  constexpr int U = 8;
+  for (int n0 = d.NT - 1; n0 >= 0; n0 -= U) {
+    float acc[U], cl[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t z = bh * d.NT + max(n0 - u, 0);
+      acc[u] = dse[(z * d.P + p) * d.N + s];
+      cl[u] = cum[(z * d.C + d.C - 1) * d.P + p];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (n0 - u < 0) break;
+      const float c = sanitize(car);
+      dse[((bh * d.NT + n0 - u) * d.P + p) * d.N + s] = c;
+      car = sanitize(c * __expf(fminf(fmaxf(cl[u], -kClipDecay), 0.f)) + acc[u]);
+    }
   }
   ds0[e] = sanitize(car);                                                                 // :219
 }
@@ -913,20 +956,36 @@ __global__ __launch_bounds__(64) void m2s_da_k(Mamba2Dims d, In dtp, int tok, co
   const float a = A[h];
   float dsum = 0.f;
   if (p < P) {
+    // U rows' loads in flight per step (every chunk length is a multiple of it)
+    constexpr int U = 8;
     float s = 0.f;
-    for (int i = 0; i < C; ++i) {                                        // :89-94
-      s += fminf(fmaxf(dt_at(i) * a, -kClipDecay), kClipDecay);
-      sCr[i][c] = s;
+    for (int i0 = 0; i0 < C; i0 += U) {                                  // :89-94
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = dt_at(i0 + u);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        s += fminf(fmaxf(v[u] * a, -kClipDecay), kClipDecay);
+        sCr[i0 + u][c] = s;
+      }
     }
     float acc = 0.f;
-    for (int i = C - 1; i >= 0; --i) {
-      const size_t o = (z * C + i) * P + p;
-      const float cr = sCr[i][c];
-      acc += dcum[o] * ((cr >= -kClipAcc && cr <= kClipAcc) ? 1.f : 0.f);   // :98,101-103
-      const float dtv = dt_at(i), raw = dtv * a;
-      const float dr = acc * ((raw >= -kClipDecay && raw <= kClipDecay) ? 1.f : 0.f);   // :106
-      ddt2[o] = sanitize(dr * a);                                        // :109,112
-      dsum = fmaf(dr, dtv, dsum);                                        // :110
+    for (int i0 = C - U; i0 >= 0; i0 -= U) {
+      float v[U], dc[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        v[u] = dt_at(i0 + u);
+        dc[u] = dcum[(z * C + i0 + u) * P + p];
+      }
+#pragma unroll
+      for (int u = U - 1; u >= 0; --u) {
+        const float cr = sCr[i0 + u][c];
+        acc += dc[u] * ((cr >= -kClipAcc && cr <= kClipAcc) ? 1.f : 0.f);   // :98,101-103
+        const float raw = v[u] * a;
+        const float dr = acc * ((raw >= -kClipDecay && raw <= kClipDecay) ? 1.f : 0.f);   // :106
+        ddt2[(z * C + i0 + u) * P + p] = sanitize(dr * a);               // :109,112
+        dsum = fmaf(dr, v[u], dsum);                                     // :110
+      }
     }
   }
 #pragma unroll
@@ -959,10 +1018,19 @@ __global__ __launch_bounds__(256) void m2s_cum_k(Mamba2Dims d, In dt, const floa
   const int n = (int)(z % d.NT), h = (int)((z / d.NT) % d.H), b = (int)(z / ((size_t)d.NT * d.H));
   const float a = A[h];
   float s = 0.f;
-  for (int i = 0; i < d.C; ++i) {
-    const size_t row = (size_t)b * d.T + (size_t)n * d.C + i;
-    s += sanitize(ld(dt, row * d.rdt + (size_t)h * d.P + p) * a, kClipDecay);
-    cum[(z * d.C + i) * d.P + p] = sanitize(s);
+  // sixteen rows' loads in flight (the chunk is a multiple of 64)
+  for (int i0 = 0; i0 < d.C; i0 += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const size_t row = (size_t)b * d.T + (size_t)n * d.C + i0 + u;
+      v[u] = ld(dt, row * d.rdt + (size_t)h * d.P + p);
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      s += sanitize(v[u] * a, kClipDecay);
+      cum[(z * d.C + i0 + u) * d.P + p] = sanitize(s);
+    }
   }
 }
 
@@ -1149,7 +1217,7 @@ int m_intra_bwd(const Mamba2Dims& d, int dtype, int dy_dtype, const void* dt, co
     hipLaunchKernelGGL(m2b_elem_k, dim3(eb), dim3(256), 0, L.st, d, idt, ix, cum, dwrite, dbx, write, d1, ddd);
   });
   if (rc != ATOMIC_OK) return rc;
-  // per-head dB = sanitize(write dstate_end)   (:57), dC = 0   (:70)
+  // per-head dB = sanitize(write dstate_end)   (:57)
   g = gemm_op(C, N, P, Z);
   g.Z1 = H; g.Z0 = NT;
   g.A = In{write, 0}; g.lda = P; g.sa = dense3((long long)C * P);
@@ -1157,9 +1225,6 @@ int m_intra_bwd(const Mamba2Dims& d, int dtype, int dy_dtype, const void* dt, co
   g.C = wB; g.ldc = N; g.sc = dense3((long long)C * N);
   g.post = 2;
   if ((rc = gemm(g, Z, "m2b_db1", L))) return rc;
-  const int fb = (int)((zcn + 255) / 256 < 65536 ? (zcn + 255) / 256 : 65536);
-  rc = L("m2b_fill", [&] { hipLaunchKernelGGL(fill0_k, dim3(fb), dim3(256), 0, L.st, wC, zcn); });
-  if (rc != ATOMIC_OK) return rc;
   const int nt16 = C / 16;
   rc = L("m2b_dbc", [&] {
     hipLaunchKernelGGL(m2b_dbc_k, dim3(nt16 * nt16, Z), dim3(256), 0, L.st, d, idy, cum, dbx, dbc);
@@ -1183,7 +1248,7 @@ int m_intra_bwd(const Mamba2Dims& d, int dtype, int dy_dtype, const void* dt, co
       g.A = In{dbc + (size_t)i0 * C + j0, 0}; g.lda = C; g.sa = dense3((long long)C * C);
       g.B = In{Bp + (size_t)j0 * d.rB * es, bf}; g.ldb = d.rB; g.sb = rows3(d.rB);
       g.C = wC + (size_t)i0 * N; g.ldc = N; g.sc = dense3((long long)C * N);
-      g.accum = 1; g.post = 2;
+      g.accum = sj > 0; g.post = 2;   // dC starts from 0 (:70)
       if ((rc = gemm(g, Z, "m2b_dc_pair", L))) return rc;
     }
   }
