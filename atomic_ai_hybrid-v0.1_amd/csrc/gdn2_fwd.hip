@@ -29,17 +29,17 @@ constexpr float kFactorLimit = 64.f;
 // ------------------------------------------------------------------ cumsum
 // Thread map for [C][K] fp32 element-wise passes: column group cg (8
 // columns), segment seg (RS consecutive rows).
-template <int C, int K>
+template <int C, int K, int NTH = 256>
 struct ColMap {
-  static constexpr int NCG = K / 8, NSEG = 256 / NCG, RS = C / NSEG;
+  static constexpr int NCG = K / 8, NSEG = NTH / NCG, RS = C / NSEG;
   static_assert(RS >= 1, "chunk too small for the thread mapping");
 };
 
 // Exclusive scan over the row segments of a ColMap pass: t holds this
 // thread's segment total for its 8 columns; out gets the sum over the lower
 // segments (REV = false) or the higher ones (REV = true).  Within a wave by
-// lane shuffles, across the 4 waves through sW (4 * K floats).
-template <int NCG, bool REV>
+// lane shuffles, across the NW waves through sW (NW * K floats).
+template <int NCG, bool REV, int NW = 4>
 __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], float* sW) {
   constexpr int SPW = 64 / NCG;  // segments per wave
   static_assert(SPW * NCG == 64, "column groups must tile a wave");
@@ -63,7 +63,7 @@ __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], 
 #pragma unroll
   for (int j = 0; j < 8; ++j) out[j] = x[j] - t[j];
 #pragma unroll
-  for (int w2 = 0; w2 < 4; ++w2)
+  for (int w2 = 0; w2 < NW; ++w2)
     if (REV ? w2 > w : w2 < w) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) out[j] += sW[w2 * NCG * 8 + cg * 8 + j];
@@ -71,15 +71,15 @@ __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], 
 }
 
 // gc = cumsum(g) over one chunk (gdn2_wy_reference.py:63) for this thread's
-// RS rows x 8 columns.  Writes gc_last to sGl[K] (sTot: NSEG*K floats of
+// RS rows x 8 columns.  Writes gc_last to sGl[K] (sTot: NTH / 64 * K floats of
 // scratch).  Returns, uniformly over the workgroup, whether the factorised
 // pairwise decay is unsafe for this chunk: some g > 0, or gc_last below
 // -kFactorLimit in some column.
-template <int C, int K>
+template <int C, int K, int NTH = 256>
 __device__ __forceinline__ bool chunk_cumsum(const float* __restrict__ g, size_t rs,
-                                             float (&gcr)[ColMap<C, K>::RS][8], float* sTot,
+                                             float (&gcr)[ColMap<C, K, NTH>::RS][8], float* sTot,
                                              float* sGl) {
-  typedef ColMap<C, K> M;
+  typedef ColMap<C, K, NTH> M;
   const int tid = threadIdx.x, cg = tid % M::NCG, seg = tid / M::NCG;
   bool positive = false;
 #pragma unroll
@@ -93,7 +93,7 @@ __device__ __forceinline__ bool chunk_cumsum(const float* __restrict__ g, size_t
 #pragma unroll
     for (int j = 0; j < 8; ++j) gcr[rr][j] += gcr[rr - 1][j];
   float off[8];
-  seg_scan8<M::NCG, false>(gcr[M::RS - 1], off, sTot);
+  seg_scan8<M::NCG, false, NTH / 64>(gcr[M::RS - 1], off, sTot);
 #pragma unroll
   for (int rr = 0; rr < M::RS; ++rr)
 #pragma unroll
@@ -112,12 +112,13 @@ __device__ __forceinline__ bool chunk_cumsum(const float* __restrict__ g, size_t
 // ------------------------------------------------------------------ layout
 template <typename T, int C, int K, int V>
 struct IntraLds {
+  static constexpr int NTH = 512, NW = NTH / 64;
   static constexpr int PAD = Pad<T>::v;
   static constexpr int LK = K + PAD, LV = V + PAD;
   static constexpr int LA = C + 4;                 // fp32 score / inverse rows
   static constexpr int LAB = C + PAD;              // operand-type inverse rows
-  static constexpr int NCG = K / 8, NSEG = 256 / NCG, RS = C / NSEG;
-  static constexpr int NCGV = V / 8, NSEGV = 256 / NCGV, RSV = C / NSEGV;
+  static constexpr int NCG = K / 8, NSEG = NTH / NCG, RS = C / NSEG;
+  static constexpr int NCGV = V / 8, NSEGV = NTH / NCGV, RSV = C / NSEGV;
   static constexpr int OPK = C * LK * (int)sizeof(T);
   static constexpr int OPV = C * LV * (int)sizeof(T);
   static constexpr int AF = C * LA * 4;
@@ -128,17 +129,19 @@ struct IntraLds {
   static constexpr int off_x = off_af + AF;                 // fp32 inverse
   static constexpr int end_a = off_x + AF;
   static constexpr int off_tot = (end_ops > end_a ? end_ops : end_a);
-  static constexpr int TOT = NSEG * K * 4;                  // cumsum segment totals; solve scratch
-  static constexpr int off_gl = off_tot + (TOT > 4 * 16 * 17 * 4 ? TOT : 4 * 16 * 17 * 4);
+  // cumsum totals of the waves; then the solve's products: two 16-row ones, one 32-row one
+  static constexpr int LT = 36, S16 = 16 * 17 * 4, SOLVE = 2 * S16 + 32 * LT * 4;
+  static constexpr int TOT = NW * K * 4 > SOLVE ? NW * K * 4 : SOLVE;
+  static constexpr int off_gl = off_tot + TOT;
   static constexpr int off_flag = off_gl + K * 4;
   static constexpr int total = off_flag + 16;
-  // phase 4 (operand-type path): per-wave [16][LS] staging of one row block of
+  // phase 4 (operand-type path): per-wave [16][64] staging of half a row block of
   // w_pseudo / u, placed over the operands that are dead by then (q, k, the
   // fp32 Akk / inverse), after the operand-type inverse
-  static constexpr int LS = (K > V ? K : V) + PAD;
+  static constexpr int LS = 64 + PAD;
   static constexpr int off_stage =
       alias_a ? ((off_af + C * (C + PAD) * (int)sizeof(T) + 15) / 16) * 16 : 0;
-  static constexpr int stage_end = off_stage + 4 * 16 * LS * (int)sizeof(T);
+  static constexpr int stage_end = off_stage + NW * 16 * LS * (int)sizeof(T);
   static constexpr bool stage_fits = stage_end <= off_b && (alias_a || stage_end <= off_af);
   static_assert(RS >= 1 && RSV >= 1, "chunk too small for the thread mapping");
   static_assert(2 * OPK >= C * K * 4, "gc scratch of the exact path must fit in sQ+sK");
@@ -146,11 +149,11 @@ struct IntraLds {
 
 // Exact pairwise scores for one chunk (reference form, used when the
 // factorised form could overflow or a positive gate breaks monotonicity).
-template <typename T, int C, int K>
+template <typename T, int C, int K, int NTH>
 __device__ void intra_scores_exact(const float* sgc, const T* q, const T* k, const T* b, size_t sq,
                                    size_t sk, size_t sb, float scale, float* out_qk, float* out_kk) {
-  // thread t computes entries e = t, t + 256, ... of the C x C matrices
-  for (int e = threadIdx.x, s = 0; e < C * C; e += 256, ++s) {
+  // thread t computes entries e = t, t + NTH, ... of the C x C matrices
+  for (int e = threadIdx.x, s = 0; e < C * C; e += NTH, ++s) {
     const int i = e / C, j = e % C;
     float aqk = 0.f, akk = 0.f;
     if (j <= i) {
@@ -182,8 +185,16 @@ __device__ void intra_scores_exact(const float* sgc, const T* q, const T* k, con
 //                   given A, all clipped to +-1e4 (kernel_c_recompute.py:46-88)
 enum { kIntraAll = 0, kIntraScores = 1, kIntraSolve = 2, kIntraRecompute = 3 };
 
+//
+// One chunk is a chain of short phases (loads and cumsum, element-wise operands,
+// scores, four 16-row substitutions, their 32- and 64-row combination, the two
+// products), so the kernel is latency, hidden by eight waves per workgroup and
+// two workgroups per CU: with four waves and a column of blocks per wave in the
+// solve, one chunk took 30k cycles (14.8 us at B1 T64 H8 K = 128, 0.383 ms at B4
+// T8192 H16), so 12.4 us and 0.330 ms, the latter 4.8 TB/s of what the kernel
+// has to move and as fast as a large copy.
 template <typename T, int C, int K, int V, int ST = kIntraAll>
-__global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __restrict__ q,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 4 : 2, 4))) void gdn2_fwd_intra(Gdn2Dims dm, const T* __restrict__ q,
                                                      const T* __restrict__ k, const T* __restrict__ v,
                                                      const T* __restrict__ w, const T* __restrict__ b,
                                                      const float* __restrict__ g, Gdn2Chunks<T> ck) {
@@ -199,6 +210,7 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
   float* sGl = reinterpret_cast<float*>(lds + L::off_gl);
   float* sGcExact = reinterpret_cast<float*>(lds + L::off_q);  // exact path only
 
+  constexpr int NTH = L::NTH, NW = L::NW;
   const int tid = threadIdx.x;
   const int bhn = blockIdx.x;
   const int n = bhn % dm.NT;
@@ -244,7 +256,7 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
   if constexpr (kRows) {
   // ---- phase 0: gc = cumsum(g) over the chunk (gdn2_wy_reference.py:63)
   float gcr[L::RS][8];
-  exact = chunk_cumsum<C, K>(gc_in, (size_t)dm.rg, gcr, sTot, sGl);
+  exact = chunk_cumsum<C, K, NTH>(gc_in, (size_t)dm.rg, gcr, sTot, sGl);
   if (kVals && tid < K) ck.gcl[(size_t)bhn * K + tid] = fin(sGl[tid]);
 
   // ---- phase 1: elementwise operands (gdn2_wy_reference.py:92-100)
@@ -308,69 +320,90 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
   const int wv_id = wave_id();
   if constexpr (kScores) {
   if (!exact) {
-    constexpr int JPW = (2 * NTRI + 3) / 4;
+    // job: 0 .. NTRI - 1 Aqk's lower tiles, then Akk's; a wave's jobs share each
+    // k step, so their MFMA chains overlap (past the last job: that one again)
+    constexpr int JPW = (2 * NTRI + NW - 1) / NW;
     f32x4 res[JPW];
+    const T* jp[JPW];
+    int jm[JPW], jn[JPW];
 #pragma unroll
     for (int cnt = 0; cnt < JPW; ++cnt) {
-      const int job = wv_id + 4 * cnt;
-      if (job >= 2 * NTRI) break;
-      const int which = job / NTRI;  // 0: Aqk, 1: Akk
+      const int job = min(wv_id + NW * cnt, 2 * NTRI - 1);
+      jp[cnt] = job / NTRI ? sB : sQ;
       int t = job % NTRI, mi = 0;
       while (t > mi) { t -= mi + 1; ++mi; }
-      const int ni = t;
-      f32x4 acc = zero4();
-      acc = tile_mma<T, false, false>(acc, which ? sB : sQ, L::LK, sK, L::LK, 16 * mi, 16 * ni, K);
+      jm[cnt] = mi;
+      jn[cnt] = t;
+      res[cnt] = zero4();
+    }
+#pragma unroll 4
+    for (int k0 = 0; k0 < K; k0 += Mma<T>::KS)
+#pragma unroll
+      for (int cnt = 0; cnt < JPW; ++cnt)
+        res[cnt] = Mma<T>::mma(Mma<T>::ld_c(jp[cnt], L::LK, 16 * jm[cnt], k0),
+                               Mma<T>::ld_c(sK, L::LK, 16 * jn[cnt], k0), res[cnt]);
+#pragma unroll
+    for (int cnt = 0; cnt < JPW; ++cnt) {
+      const bool kk = min(wv_id + NW * cnt, 2 * NTRI - 1) >= NTRI;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * mi + tile_row(i), c = 16 * ni + tile_col();
-        float x = which ? acc[i] : dm.scale * acc[i];
-        const bool keep = which ? (r > c) : (r >= c);
-        acc[i] = keep ? n2n(x) : 0.f;
+        const int r = 16 * jm[cnt] + tile_row(i), c = 16 * jn[cnt] + tile_col();
+        const float x = kk ? res[cnt][i] : dm.scale * res[cnt][i];
+        const bool keep = kk ? (r > c) : (r >= c);
+        res[cnt][i] = keep ? n2n(x) : 0.f;
       }
-      res[cnt] = acc;
     }
     __syncthreads();  // sQ / sK are dead from here on; sAf may alias them
 #pragma unroll
     for (int cnt = 0; cnt < JPW; ++cnt) {
-      const int job = wv_id + 4 * cnt;
+      const int job = wv_id + NW * cnt;
       if (job >= 2 * NTRI) break;
-      const int which = job / NTRI;
-      int t = job % NTRI, mi = 0;
-      while (t > mi) { t -= mi + 1; ++mi; }
-      const int ni = t;
-      if (which == 0) store_tile_n(g_aqk, C, 16 * mi, 16 * ni, res[cnt]);
-      else if constexpr (ST == kIntraScores) store_tile_n(g_akk, C, 16 * mi, 16 * ni, res[cnt]);
-      else store_tile_n(sAf, L::LA, 16 * mi, 16 * ni, res[cnt]);
+      if (job < NTRI) store_tile_n(g_aqk, C, 16 * jm[cnt], 16 * jn[cnt], res[cnt]);
+      else if constexpr (ST == kIntraScores) store_tile_n(g_akk, C, 16 * jm[cnt], 16 * jn[cnt], res[cnt]);
+      else store_tile_n(sAf, L::LA, 16 * jm[cnt], 16 * jn[cnt], res[cnt]);
     }
   } else {
-    constexpr int PER = C * C / 256;
+    constexpr int PER = C * C / NTH;
     float eqk[PER], ekk[PER];
-    intra_scores_exact<T, C, K>(sGcExact, qc, kc, bc, dm.rq, dm.rk, dm.rb, dm.scale, eqk, ekk);
+    intra_scores_exact<T, C, K, NTH>(sGcExact, qc, kc, bc, dm.rq, dm.rk, dm.rb, dm.scale, eqk, ekk);
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < PER; ++s) {
-      const int e = tid + 256 * s, i = e / C, j = e % C;
+      const int e = tid + NTH * s, i = e / C, j = e % C;
       g_aqk[i * C + j] = from_f<T>(eqk[s]);
       if constexpr (ST == kIntraScores) g_akk[i * C + j] = from_f<T>(ekk[s]);
       else sAf[i * L::LA + j] = ekk[s];
     }
   }
-  // upper tiles of Aqk / Akk are zero
-  for (int e = tid; e < C * C; e += 256) {
-    const int i = e / C, j = e % C;
-    if ((j >> 4) > (i >> 4)) {
-      if (!exact) g_aqk[i * C + j] = from_f<T>(0.f);
-      if constexpr (ST == kIntraScores) g_akk[i * C + j] = from_f<T>(0.f);
-      else sAf[i * L::LA + j] = 0.f;
+  // upper tiles of Aqk / Akk are zero (in LDS only the lower blocks of Akk are
+  // read), and so is the inverse until its blocks are written; 16 bytes an item
+  // where the caller's array allows it
+  const u32x4 z4 = {0u, 0u, 0u, 0u};
+  auto zero_upper = [&](T* p) {
+    constexpr int VC = 16 / (int)sizeof(T);
+    const bool wide = (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+    for (int e = tid; e < C * C / VC; e += NTH) {
+      const int i = e / (C / VC), j = (e % (C / VC)) * VC;
+      if ((j >> 4) <= (i >> 4)) continue;
+      if (wide) {
+        *reinterpret_cast<u32x4*>(p + i * C + j) = z4;
+      } else {
+#pragma unroll
+        for (int t = 0; t < VC; ++t) p[i * C + j + t] = from_f<T>(0.f);
+      }
     }
-    if constexpr (ST == kIntraAll) sX[i * L::LA + j] = 0.f;
-  }
+  };
+  if (!exact) zero_upper(g_aqk);
+  if constexpr (ST == kIntraScores) zero_upper(g_akk);
+  if constexpr (ST == kIntraAll)
+    for (int e = tid; e < C * C / 4; e += NTH)
+      *reinterpret_cast<u32x4*>(sX + e / (C / 4) * L::LA + (e % (C / 4)) * 4) = z4;
   if constexpr (ST == kIntraScores) return;
   __syncthreads();
   }  // kScores
   if constexpr (ST == kIntraSolve) {
     // Akk from the caller (only its strictly lower blocks are read below)
-    for (int e = tid; e < C * C; e += 256) {
+    for (int e = tid; e < C * C; e += NTH) {
       const int i = e / C, j = e % C;
       sAf[i * L::LA + j] = to_f(g_akk[i * C + j]);
       sX[i * L::LA + j] = 0.f;
@@ -383,49 +416,64 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
   const T* opA;
   int ldA;
   if constexpr (ST != kIntraRecompute) {
+  static_assert(C == 64 && NW >= 4, "two levels of 2 x 2 blocks over 16-row blocks");
   // Diagonal 16x16 blocks by forward substitution (wave w, lane = column).
   {
     const int lane = lane_id();
     if (wv_id < NB && lane < 16) {
       const int o = 16 * wv_id;
+      f32x4 row[16][4];  // the block's rows, every lane the same
+#pragma unroll
+      for (int i = 1; i < 16; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (4 * q < i) row[i][q] = *reinterpret_cast<const f32x4*>(sAf + (o + i) * L::LA + o + 4 * q);
       float x[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float s = (i == lane) ? 1.f : 0.f;
+      for (int i = 0; i < 16; ++i) x[i] = (i == lane) ? 1.f : 0.f;
 #pragma unroll
-        for (int j = 0; j < 15; ++j)  // constant trip count: x stays in registers
-          if (j < i) s -= sAf[(o + i) * L::LA + o + j] * x[j];
-        x[i] = s;
-      }
+      for (int j = 0; j < 15; ++j)  // x_j is final: into every later row
+#pragma unroll
+        for (int i = j + 1; i < 16; ++i) x[i] -= row[i][j / 4][j % 4] * x[j];
 #pragma unroll
       for (int i = 0; i < 16; ++i) sX[(o + i) * L::LA + o + lane] = x[i];
     }
   }
   __syncthreads();
-  // Off-diagonal blocks, one column block per wave:
-  //   A_mn = -A_mm (sum_{k=n}^{m-1} T_mk A_kn)
-  {
-    float* scr = sTot + wv_id * 16 * 17;
-    for (int nb = wv_id; nb < NB; nb += 4) {
-      for (int mb = nb + 1; mb < NB; ++mb) {
-        f32x4 acc = zero4();
-        acc = tile_mma<float, false, true>(acc, sAf + 16 * nb, L::LA, sX + 16 * nb * L::LA, L::LA,
-                                           16 * mb, 16 * nb, 16 * (mb - nb));
-        store_tile_n(scr, 17, 0, 0, acc);
-        wave_lds_sync();  // scr is private to this wave
-        f32x4 a2 = zero4();
-        a2 = tile_mma<float, false, true>(a2, sX + 16 * mb * L::LA + 16 * mb, L::LA, scr, 17, 0, 0, 16);
+  // [[A0, 0], [-A1 T A0, A1]] of two 16-row blocks for both 32-row halves
+  if (wv_id < 2) {
+    const int o = 32 * wv_id;
+    float* scr = sTot + wv_id * (L::S16 / 4);  // private to this wave
+    const f32x4 p = tile_mma<float, false, true>(zero4(), sAf + o, L::LA, sX + o * L::LA + o, L::LA, o + 16, 0, 16);
+    store_tile_n(scr, 17, 0, 0, p);
+    wave_lds_sync();
+    f32x4 a = tile_mma<float, false, true>(zero4(), sX + (o + 16) * L::LA + o + 16, L::LA, scr, 17, 0, 0, 16);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a2[i] = -a2[i];
-        store_tile_n(sX, L::LA, 16 * mb, 16 * nb, a2);
-      }
-    }
+    for (int i = 0; i < 4; ++i) a[i] = -a[i];
+    store_tile_n(sX, L::LA, o + 16, o, a);
+  }
+  __syncthreads();
+  // the same of the two halves: a 16 x 16 tile (m, n) per wave, over the nonzero blocks
+  float* s32 = sTot + 2 * (L::S16 / 4);
+  const int tm = (wv_id >> 1) & 1, tn = wv_id & 1;
+  if (wv_id < 4) {
+    const f32x4 p = tile_mma<float, false, true>(zero4(), sAf + 16 * tn, L::LA, sX + 16 * tn * L::LA, L::LA,
+                                                 32 + 16 * tm, 16 * tn, 32 - 16 * tn);
+    store_tile_n(s32, L::LT, 16 * tm, 16 * tn, p);
+  }
+  __syncthreads();
+  if (wv_id < 4) {
+    f32x4 a = tile_mma<float, false, true>(zero4(), sX + 32 * L::LA + 32, L::LA, s32, L::LT, 16 * tm, 16 * tn,
+                                           16 + 16 * tm);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = -a[i];
+    store_tile_n(sX, L::LA, 32 + 16 * tm, 16 * tn, a);
   }
   __syncthreads();
   // n2n, operand-type copy, global A
   if constexpr (sizeof(T) == 2) {
     T* sAb = reinterpret_cast<T*>(lds + L::off_af);  // Akk is dead
-    for (int e = tid; e < C * C / 8; e += 256) {  // 8 consecutive columns per item
+    for (int e = tid; e < C * C / 8; e += NTH) {  // 8 consecutive columns per item
       const int i = e / (C / 8), j = (e % (C / 8)) * 8;
       float x[8];
       load8(sX + i * L::LA + j, x);
@@ -437,7 +485,7 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
     opA = sAb;
     ldA = C + Pad<T>::v;
   } else {
-    for (int e = tid; e < C * C; e += 256) {
+    for (int e = tid; e < C * C; e += NTH) {
       const int i = e / C, j = e % C;
       const float x = n2n(sX[i * L::LA + j]);
       sX[i * L::LA + j] = x;
@@ -451,7 +499,7 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
     // A from the caller, into the operand-type rows phase 4 reads
     if constexpr (sizeof(T) == 2) {
       T* sAb = reinterpret_cast<T*>(lds + L::off_af);
-      for (int e = tid; e < C * C / 8; e += 256) {
+      for (int e = tid; e < C * C / 8; e += NTH) {
         const int i = e / (C / 8), j = (e % (C / 8)) * 8;
         *reinterpret_cast<uint4*>(sAb + i * (C + Pad<T>::v) + j) =
             *reinterpret_cast<const uint4*>(g_ainv + i * C + j);
@@ -459,7 +507,7 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
       opA = sAb;
       ldA = C + Pad<T>::v;
     } else {
-      for (int e = tid; e < C * C; e += 256) {
+      for (int e = tid; e < C * C; e += NTH) {
         const int i = e / C, j = e % C;
         sX[i * L::LA + j] = g_ainv[i * C + j];
       }
@@ -473,56 +521,59 @@ __global__ __launch_bounds__(256) void gdn2_fwd_intra(Gdn2Dims dm, const T* __re
   T* g_wt = ck.wt + (size_t)bhn * C * K;
   T* g_u = ck.u + (size_t)bhn * C * V;
   if constexpr (sizeof(T) == 2 && L::stage_fits) {
-    // one row block per wave: its column tiles share the A reads, go through
-    // the wave's LDS staging rows and leave as 16-byte row pieces
+    // waves 0-3 a row block of w_pseudo each, 4-7 of u: 64 columns at a time, whose
+    // tiles share the A reads, go through the wave's LDS staging rows and
+    // leave as 16-byte row pieces
+    static_assert(NW == 2 * NB && K == V, "a row block of each product per wave");
     T* stg = reinterpret_cast<T*>(lds + L::off_stage) + wv_id * 16 * L::LS;
-    auto row_block = [&](int mi, int kr, const T* Bop, int ldb, auto ncol, T* gout) {
-      constexpr int NC = decltype(ncol)::value;
-      f32x4 acc[NC / 16];
+    const int mi = wv_id % NB;
+    const bool isu = wv_id >= NB;
+    const T* Bop = isu ? sW : sB;
+    T* gout = (isu ? g_u : g_wt) + (size_t)16 * mi * K;
+    // A is block lower triangular; a caller's A (kernel C alone) is read whole
+    int kr = ST == kIntraRecompute ? C : 16 * (mi + 1);
+    kr = ((kr + Mma<T>::KS - 1) / Mma<T>::KS) * Mma<T>::KS;
+    if (kr > C) kr = C;
 #pragma unroll
-      for (int t = 0; t < NC / 16; ++t) acc[t] = zero4();
-      tile_mma_row<T, false, true, NC / 16>(acc, opA, ldA, Bop, ldb, 16 * mi, 0, kr);
+    for (int c0 = 0; c0 < K; c0 += 64) {
+      f32x4 acc[4];
 #pragma unroll
-      for (int t = 0; t < NC / 16; ++t) {
+      for (int t = 0; t < 4; ++t) acc[t] = zero4();
+      tile_mma_row<T, false, true, 4>(acc, opA, ldA, Bop, L::LK, 16 * mi, c0, kr);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[t][i] = fin(acc[t][i]);
         store_tile_n(stg, L::LS, 0, 16 * t, acc[t]);
       }
       wave_lds_sync();
-      constexpr int PR = NC / 8;  // 16-byte pieces per row
 #pragma unroll
-      for (int e = lane_id(); e < 16 * PR; e += 64) {
-        const int r = e / PR, c = (e % PR) * 8;
-        *reinterpret_cast<uint4*>(gout + (size_t)(16 * mi + r) * NC + c) =
-            *reinterpret_cast<const uint4*>(stg + r * L::LS + c);
+      for (int e = lane_id(); e < 16 * 8; e += 64) {
+        const int r = e / 8, c = (e % 8) * 8;
+        *reinterpret_cast<uint4*>(gout + (size_t)r * K + c0 + c) = *reinterpret_cast<const uint4*>(stg + r * L::LS + c);
       }
       wave_lds_sync();  // the staging rows are rewritten next
-    };
-    for (int mi = wv_id; mi < NB; mi += 4) {
-      // A is block lower triangular; a caller's A (kernel C alone) is read whole
-      int kr = ST == kIntraRecompute ? C : 16 * (mi + 1);
-      kr = ((kr + Mma<T>::KS - 1) / Mma<T>::KS) * Mma<T>::KS;
-      if (kr > C) kr = C;
-      row_block(mi, kr, sB, L::LK, std::integral_constant<int, K>(), g_wt);
-      row_block(mi, kr, sW, L::LV, std::integral_constant<int, V>(), g_u);
     }
   } else {
-    constexpr int TW = NB * (K / 16), TU = NB * (V / 16);
-    for (int job = wv_id; job < TW + TU; job += 4) {
-      const bool isu = job >= TW;
-      const int jj = isu ? job - TW : job;
-      const int nbk = isu ? V / 16 : K / 16;
-      const int mi = jj / nbk, ni = jj % nbk;
-      int kr = ST == kIntraRecompute ? C : 16 * (mi + 1);
-      kr = ((kr + Mma<T>::KS - 1) / Mma<T>::KS) * Mma<T>::KS;
-      if (kr > C) kr = C;
-      f32x4 acc = zero4();
-      if (isu) acc = tile_mma<T, false, true>(acc, opA, ldA, sW, L::LV, 16 * mi, 16 * ni, kr);
-      else acc = tile_mma<T, false, true>(acc, opA, ldA, sB, L::LK, 16 * mi, 16 * ni, kr);
-  #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = fin(acc[i]);
-      if (isu) store_tile_n(g_u, V, 16 * mi, 16 * ni, acc);
-      else store_tile_n(g_wt, K, 16 * mi, 16 * ni, acc);
+    // a row block of w_pseudo or u per wave, its column tiles four at a time (their
+    // MFMA chains overlap)
+    static_assert(NW == 2 * NB && K == V, "a row block of each product per wave");
+    const int mi = wv_id % NB;
+    const bool isu = wv_id >= NB;
+    int kr = ST == kIntraRecompute ? C : 16 * (mi + 1);
+    kr = ((kr + Mma<T>::KS - 1) / Mma<T>::KS) * Mma<T>::KS;
+    if (kr > C) kr = C;
+    for (int c0 = 0; c0 < K; c0 += 64) {
+      f32x4 acc[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t] = zero4();
+      tile_mma_row<T, false, true, 4>(acc, opA, ldA, isu ? sW : sB, L::LK, 16 * mi, c0, kr);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][i] = fin(acc[t][i]);
+        store_tile_n(isu ? g_u : g_wt, K, 16 * mi, c0 + 16 * t, acc[t]);
+      }
     }
   }
 }

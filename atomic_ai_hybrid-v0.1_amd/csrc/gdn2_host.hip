@@ -174,7 +174,7 @@ static int gdn2_intra_launch(const Gdn2Plan& p, const void* q, const void* k, co
   hipStream_t st = L.st;
   static const char* const names[] = {"gdn2_fwd_intra", "gdn2_chunk_scores", "gdn2_wy_solve", "gdn2_recompute_wy"};
   return L(names[ST], [&] {
-    hipLaunchKernelGGL((gdn2_fwd_intra<T, C, K, V, ST>), dim3((unsigned)p.bhn), dim3(256), 0, st, p.dm,
+    hipLaunchKernelGGL((gdn2_fwd_intra<T, C, K, V, ST>), dim3((unsigned)p.bhn), dim3(512), 0, st, p.dm,
                        (const T*)q, (const T*)k, (const T*)v, (const T*)w, (const T*)b, g, ck);
   });
 }
