@@ -269,6 +269,21 @@ __device__ __forceinline__ void dma_touch(const void* src, void* dst) {
   typedef __attribute__((address_space(3))) uint32_t* lp;
   __builtin_amdgcn_global_load_lds((gp)(uintptr_t)src, (lp)(uint32_t)(uintptr_t)dst, 4, 0, 0);
 }
+// The same load for waves that also read LDS: the compiler does not see it, so it
+// does not wait for it before every LDS read that may alias; the wave waits
+// with vm_wait before the barrier that publishes it.  dst from lds_addr.
+__device__ __forceinline__ void dma16_raw(const void* src, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+// At most N vector-memory operations outstanding (loads complete in order, so
+// operations the compiler issued in between only make this wait longer).
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 // A workgroup barrier that does not wait for the wave's own outstanding memory
 // operations (a loader wave keeps its loads in flight across it).
 __device__ __forceinline__ void bare_barrier() {

@@ -8,7 +8,8 @@
 //   gemm_tn   P[s][K][N] = sum over the rows m of split s of X[m][K] D[m][N]
 //             (the weight gradient X^T D over the tokens), fp32 partials.
 //
-// Tiles: one 128 x BN block of C per workgroup of four waves (2 x 2, each
+// Tiles: 256 x 256 per workgroup of eight waves where the sizes allow (the _big
+// kernels); else one 128 x BN block of C per workgroup of four waves (2 x 2, each
 // 64 x BN/2 as v_mfma_f32_16x16x32_bf16 tiles; BN = 256 where N allows, else
 // 128); the reduction dimension in steps of 64 through one LDS stage: the
 // next step's 16-byte pieces are loaded into registers while the current
@@ -147,6 +148,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   epi(tm * kGT + wm, tn * BN + wn, acc);
 }
 
+// 256 x 256 tiles, one workgroup of eight waves per CU (each 128 x 64), the
+// reduction in steps of 32 through four LDS stages that the waves load without
+// registers three steps ahead; one barrier a step.  Per CU a step reads 96 KB
+// of fragments for 1024 cycles of MFMA per SIMD.  Stage rows of 64 bytes, their
+// four pieces permuted by (row / 4) & 3 (in the loads' global addresses), so
+// that a fragment read meets no bank conflict.  Bit-identical to gemm_nt.
+// M 32768, bf16 result: 1792 x 1536 0.271 -> 0.239 ms (754 TFLOP/s; 3.5 rounds of
+// tiles), 1536 x 1792 0.262 -> 0.215 (839); with their epilogues 0.330 -> 0.282
+// and 0.272 -> 0.230.  Two alternating groups of waves
+// (one reading LDS, one on MFMA) gave 2 % more here and less in gemm_tn_big.
+constexpr int kBigT = 256, kBigK = 32, kBigS = 4;
+
+template <typename Epi>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_nt_big(GemmNT g, Epi epi) {
+  constexpr int SB = kBigT * kBigK * 2;   // bytes of one operand's stage
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kBigS * 2 * SB];
+  const int w = wave_id(), lane = lane_id();
+  int tm, tn;
+  xcd_group_map(blockIdx.x, g.M / kBigT, g.N / kBigT, tm, tn);
+  const int nk = g.K / kBigK;
+  // this wave's four loads of a stage: 16 rows of 64 bytes each (waves 0-3 A, 4-7 B)
+  const bool isb = w >= 4;
+  const bf16* base = isb ? g.Bt + (size_t)tn * kBigT * g.ldb : g.A + (size_t)tm * kBigT * g.lda;
+  const long long ld = isb ? g.ldb : g.lda;
+  const char* src[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 64 * (w & 3) + 16 * i + (lane >> 2);
+    const int piece = (lane & 3) ^ ((row >> 2) & 3);
+    src[i] = reinterpret_cast<const char*>(base + (size_t)row * ld + piece * 8);
+  }
+  const uint32_t l0 = lds_addr(lds) + (isb ? SB : 0) + (w & 3) * 4096;
+  auto issue = [&](int t) {
+    const uint32_t d = l0 + (t % kBigS) * 2 * SB;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16_raw(src[i] + (size_t)t * (kBigK * 2), d + i * 1024);
+  };
+  f32x4 acc[2][4][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][i][j] = zero4();
+  const int wm = 128 * (w >> 2), wn = 64 * (w & 3);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int fo = r16 * 64 + ((g4 ^ ((r16 >> 2) & 3)) * 16);   // a fragment row's 16 bytes within its 16 rows
+  issue(0); issue(1); issue(2);
+  for (int t = 0; t < nk; ++t) {
+    if (t + 2 < nk) vm_wait<8>();
+    else vm_wait<0>();
+    bare_barrier();
+    if (t + 3 < nk) issue(t + 3);
+    const unsigned char* sA = lds + (t % kBigS) * 2 * SB + wm * 64 + fo;
+    const unsigned char* sB = lds + (t % kBigS) * 2 * SB + SB + wn * 64 + fo;
+    bf16x8 bf[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(sB + j * 1024);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bf16x8 af = *reinterpret_cast<const bf16x8*>(sA + (4 * h + i) * 1024);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[h][i][j] = Mma<bf16>::mma(af, bf[j], acc[h][i][j]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the stage are done
+  }
+  // The epilogue takes whole 16-byte row pieces (four consecutive lanes of an MFMA
+  // tile hold four rows, and stored from there a wave wrote 32 bytes of each of
+  // 16 rows: the forward 0.335 ms): each wave's 64 x 64 halves pass through LDS as bf16.
+  __syncthreads();  // the last stage is read
+  bf16* st = reinterpret_cast<bf16*>(lds) + w * 64 * 72;
+  const int c = tile_col();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float v[4] = {acc[h][i][j][0], acc[h][i][j][1], acc[h][i][j][2], acc[h][i][j][3]};
+        quad_transpose(v);
+        st4bf(st + (16 * i + tile_row(0) + (c & 3)) * 72 + 16 * j + (c & ~3), v);
+      }
+    wave_lds_sync();
+#pragma unroll 2
+    for (int p = 0; p < 8; ++p) {
+      const int r = 8 * p + (lane >> 3), cc = 8 * (lane & 7);
+      float v[8];
+      load8(st + r * 72 + cc, v);
+      epi.row8(tm * kBigT + wm + 64 * h + r, tn * kBigT + wn + cc, v);
+    }
+    wave_lds_sync();  // the rows are rewritten next
+  }
+}
+
 // ---------------------------------------------------------------- TN GEMM
 struct GemmTN {
   const bf16* X;  // [M][Kd], row stride ldx
@@ -154,8 +251,10 @@ struct GemmTN {
   const bf16* D;  // [M][N], row stride ldd
   long long ldd;
   int Kd, N;      // multiples of 128 and BN
-  int rows;       // rows per split (a multiple of 64); split s covers rows [s rows, (s + 1) rows)
+  int rows;       // rows per split (a multiple of 64; 32 in gemm_tn_big); split s covers
+                  // rows [s rows, (s + 1) rows), in gemm_tn_big no further than M
   float* part;    // [splits][Kd][N]
+  int M;
 };
 
 // P[s] tile (128 x BN) = X^T D over the split's rows, both operands staged as
@@ -243,6 +342,86 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+// The same in 256 x 256 tiles (see gemm_nt_big): stages of 32 rows of 512 bytes of
+// each operand, read transposed; their 16-byte pieces are permuted so that the
+// eight rows a half wave reads together lie 32 bytes apart in the banks.
+// 1536 x 1792 over 32768 rows: 0.309 -> 0.206 ms (876 TFLOP/s, six splits).
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tn_big(GemmTN g) {
+  constexpr int SB = kBigT * kBigK * 2;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kBigS * 2 * SB];
+  const int w = wave_id(), lane = lane_id();
+  const int ntn = g.N / kBigT, ntk = g.Kd / kBigT;
+  // the tiles of one split share its rows: splits over the XCDs
+  const int tiles = ntk * ntn;
+  const int s = blockIdx.x / tiles, tt = blockIdx.x % tiles;
+  const int tk = tt / ntn, tn = tt % ntn;
+  const int m0 = s * g.rows, m1 = min(m0 + g.rows, g.M);
+  const int nk = (m1 - m0) / kBigK;
+  const bool isb = w >= 4;
+  const bf16* base = isb ? g.D + (size_t)m0 * g.ldd + tn * kBigT : g.X + (size_t)m0 * g.ldx + tk * kBigT;
+  const long long ld = isb ? g.ldd : g.ldx;
+  auto swz = [](int row) { return 2 * ((row & 3) | (((row >> 3) & 1) << 2)); };
+  const char* src[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {   // two rows of 512 bytes each
+    const int row = 8 * (w & 3) + 2 * i + (lane >> 5);
+    src[i] = reinterpret_cast<const char*>(base + (size_t)row * ld + (((lane & 31) ^ swz(row)) * 8));
+  }
+  const size_t adv = (size_t)kBigK * ld * 2;
+  const uint32_t l0 = lds_addr(lds) + (isb ? SB : 0) + (w & 3) * 4096;
+  auto issue = [&](int t) {
+    const uint32_t d = l0 + (t % kBigS) * 2 * SB;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16_raw(src[i] + (size_t)t * adv, d + i * 1024);
+  };
+  f32x4 acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = zero4();
+  const int wm = 128 * (w >> 2), wn = 64 * (w & 3);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  typedef __attribute__((address_space(3))) bf16x4* lds_p;
+  auto frag = [&](const unsigned char* st, int c0) {   // (k = row, i = column c0 + r16)
+    const int row = 8 * g4 + (r16 >> 2);
+    const int pc = (c0 >> 3) + ((r16 & 3) >> 1), by = (r16 & 1) * 8;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_p)(st + row * 512 + ((pc ^ swz(row)) * 16) + by));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_p)(st + (row + 4) * 512 + ((pc ^ swz(row + 4)) * 16) + by));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  for (int t = 0; t < 3 && t < nk; ++t) issue(t);
+  for (int t = 0; t < nk; ++t) {
+    if (t + 2 < nk) vm_wait<8>();
+    else vm_wait<0>();
+    bare_barrier();
+    if (t + 3 < nk) issue(t + 3);
+    const unsigned char* sX = lds + (t % kBigS) * 2 * SB;
+    const unsigned char* sD = sX + SB;
+    bf16x8 bf[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bf[j] = frag(sD, wn + 16 * j);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bf16x8 af = frag(sX, wm + 16 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = Mma<bf16>::mma(af, bf[j], acc[i][j]);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  float* P = g.part + (size_t)s * g.Kd * g.N;
+  const int c = tile_col();
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+      quad_transpose(v);
+      const int row = tk * kBigT + wm + 16 * i + tile_row(0) + (c & 3);
+      const int col = tn * kBigT + wn + 16 * j + (c & ~3);
+      *reinterpret_cast<float4*>(P + (size_t)row * g.N + col) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
 // ---------------------------------------------------------------- epilogues
 __device__ __forceinline__ float m2p_dt_lo() { return bf16r(1e-2f); }
 // jax.nn.softplus(x) = logaddexp(x, 0); every use rounds the result to bf16
@@ -262,6 +441,29 @@ struct M2ProjEpi {
   const float* b_dt;               // [d]
   bf16 *dt, *B, *C;                // [M][d], [M][n], [M][n]
   bf16 *dt_pre, *b_pre, *c_pre;    // the same shapes, or NULL
+  // eight columns of one row, the products rounded to bf16 (all outputs 16-byte aligned)
+  __device__ __forceinline__ void row8(int row, int col, float (&v)[8]) const {
+    float o[8];
+    if (col < d) {  // uniform over a wave's 64 columns
+      float bv[8];
+      load8(b_dt + col, bv);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[k] = bf16r(v[k] + bf16r(bv[k]));
+        o[k] = m2p_sanit(fminf(fmaxf(bf16r(m2p_softplus(v[k])), m2p_dt_lo()), 1.f), 1e3f);
+      }
+      store8(dt + (size_t)row * d + col, o);
+      if (dt_pre) store8(dt_pre + (size_t)row * d + col, v);
+    } else {
+      const bool isb = col < d + n;
+      const int cc = isb ? col - d : col - d - n;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o[k] = m2p_sanit(v[k], 1e3f);
+      store8((isb ? B : C) + (size_t)row * n + cc, o);
+      bf16* pre = isb ? b_pre : c_pre;
+      if (pre) store8(pre + (size_t)row * n + cc, v);
+    }
+  }
   template <int NJ>
   __device__ __forceinline__ void operator()(int m0, int n0, f32x4 (&acc)[4][NJ]) const {
     const int c = tile_col();
@@ -310,6 +512,13 @@ struct M2DxEpi {
   int d;
   bf16* out;        // [M] rows of stride ldo
   long long ldo;
+  __device__ __forceinline__ void row8(int row, int col, float (&v)[8]) const {
+    float cv[8];
+    load8(dxc + (size_t)row * d + col, cv);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] += cv[k];
+    store8(out + (size_t)row * ldo + col, v);
+  }
   template <int NJ>
   __device__ __forceinline__ void operator()(int m0, int n0, f32x4 (&acc)[4][NJ]) const {
     const int c = tile_col();
@@ -377,53 +586,60 @@ __device__ __forceinline__ float m2p_range_g(float x, float lo, float hi) {
 }
 
 // The element-wise VJP of M2ProjEpi into dPre [M][d + 2n] (columns: dt, B, C
-// pre-activations), one thread per 8 columns of 32 rows; column sums of the
+// pre-activations), one thread per 4 columns of 32 rows; column sums of the
 // dt part (b_dt's gradient) per 32 rows into dbpart [M / 32][d].  Block 0
 // also writes dA_log from dA (A = -exp(clip(A_log, +-20)), model.py:420-422).
+// Its four transcendentals an element and its 6 bytes take about as long as each
+// other: softplus and its derivative share one exponential, the loads of
+// eight rows are in flight together, and 4 columns a thread give seven waves per
+// SIMD (8 columns, two exponentials: 0.142 ms at 32768 x 1792, now 0.105).
 __global__ __launch_bounds__(256) void m2p_vjp(int M, int d, int n, int H, const bf16* __restrict__ dt_pre,
                                                const bf16* __restrict__ b_pre, const bf16* __restrict__ c_pre,
                                                const float* __restrict__ a_log, const bf16* __restrict__ ddt,
                                                const bf16* __restrict__ dB, const bf16* __restrict__ dC,
                                                const float* __restrict__ dA, bf16* __restrict__ dpre,
                                                float* __restrict__ dbpart, float* __restrict__ da_log) {
-  const int nt = d + 2 * n, ncg = nt / 8;
+  const int nt = d + 2 * n, ncg = nt / 4;
   const size_t gi = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (gi < (size_t)(M / 32) * ncg) {
     const int cg = (int)(gi % ncg), rt = (int)(gi / ncg);
-    const int col = cg * 8;
-    if (col < d) {
-      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int r = 0; r < 32; ++r) {
-        const size_t m = (size_t)rt * 32 + r;
-        float v[8], g[8], o[8];
-        load8(dt_pre + m * d + col, v);
-        load8(ddt + m * d + col, g);
+    const int col = cg * 4;
+    constexpr int U = 8;
+    const bool isdt = col < d, isb = col < d + n;
+    const int cc = isdt ? col : (isb ? col - d : col - d - n), ld = isdt ? d : n;
+    const bf16* pre = (isdt ? dt_pre : (isb ? b_pre : c_pre)) + cc;
+    const bf16* gg = (isdt ? ddt : (isb ? dB : dC)) + cc;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int r0 = 0; r0 < 32; r0 += U) {
+      bf16x4 rv[U], rg[U];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float sp = bf16r(m2p_softplus(v[j]));
-          const float cl = fminf(fmaxf(sp, m2p_dt_lo()), 1.f);
-          const float dsp = bf16r(g[j] * m2p_clip_g(cl, 1e3f) * m2p_range_g(sp, m2p_dt_lo(), 1.f));
-          o[j] = bf16r(dsp * __builtin_amdgcn_rcpf(1.f + __expf(-v[j])));  // softplus' = logistic
-          acc[j] += o[j];
-        }
-        store8(dpre + m * nt + col, o);
+      for (int u = 0; u < U; ++u) {
+        const size_t m = (size_t)rt * 32 + r0 + u;
+        rv[u] = *reinterpret_cast<const bf16x4*>(pre + m * ld);
+        rg[u] = *reinterpret_cast<const bf16x4*>(gg + m * ld);
       }
-      store8(dbpart + (size_t)rt * d + col, acc);
-    } else {
-      const bool isb = col < d + n;
-      const int cc = isb ? col - d : col - d - n;
-      const bf16* pre = isb ? b_pre : c_pre;
-      const bf16* gg = isb ? dB : dC;
-      for (int r = 0; r < 32; ++r) {
-        const size_t m = (size_t)rt * 32 + r;
-        float v[8], g[8], o[8];
-        load8(pre + m * n + cc, v);
-        load8(gg + m * n + cc, g);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = bf16r(g[j] * m2p_clip_g(v[j], 1e3f));
-        store8(dpre + m * nt + col, o);
+      for (int u = 0; u < U; ++u) {
+        float o[4];
+        if (isdt) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float v = (float)rv[u][j], e = __expf(-fabsf(v));
+            const float sp = bf16r(fmaxf(v, 0.f) + __logf(1.f + e));   // m2p_softplus
+            // the clip to [lo, 1] keeps its result inside the +-1e3 of the sanitise after it
+            const float dsp = bf16r((float)rg[u][j] * m2p_range_g(sp, m2p_dt_lo(), 1.f));
+            const float ri = __builtin_amdgcn_rcpf(1.f + e);
+            o[j] = bf16r(dsp * (v >= 0.f ? ri : e * ri));  // softplus' = logistic
+            acc[j] += o[j];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = bf16r((float)rg[u][j] * m2p_clip_g((float)rv[u][j], 1e3f));
+        }
+        st4bf(dpre + ((size_t)rt * 32 + r0 + u) * nt + col, o);
       }
     }
+    if (isdt) *reinterpret_cast<float4*>(dbpart + (size_t)rt * d + col) = make_float4(acc[0], acc[1], acc[2], acc[3]);
   }
   if (blockIdx.x == 0)
     for (int h = threadIdx.x; h < H; h += 256) {

@@ -21,6 +21,8 @@
 // three following cotangents, recomputed past the tile's end).  Parameter
 // gradients: each workgroup (four consecutive tiles) combines its waves'
 // sums through LDS into one partial row; a final kernel sums the rows.
+#include <initializer_list>
+
 #include "../../include/atomic_hybrid.h"
 #include "common.hpp"
 #include "launch.hpp"
@@ -824,9 +826,27 @@ static int m2x_check(const atomic_mamba2_proj_args* a) {
 // partials [M / 32][d] and sums [d] fp32, and the convolution's partial rows.
 struct M2xPlan {
   PlDims dm;
-  int M, d, n, nt, splits;
+  int M, d, n, nt, splits, rows;
+  bool dw_big;
   size_t o_w, o_dpre, o_dxc, o_dw, o_dbp, o_dbs, o_conv, o_convsum, total;
 };
+static bool aligned16(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (reinterpret_cast<uintptr_t>(p) & 15) return false;
+  return true;
+}
+// C = A Bt^T over rows: 256 x 256 tiles where both sides divide and there are
+// more than 128 of them (with fewer, twice as many workgroups of 128 x 256
+// leave less of the chip idle) and the outputs take 16-byte stores.
+template <typename Epi>
+static void m2x_gemm_nt(const GemmNT& g, const Epi& e, bool aligned, hipStream_t st) {
+  if (aligned && g.M % kBigT == 0 && g.N % kBigT == 0 && (g.M / kBigT) * (g.N / kBigT) > 128)
+    hipLaunchKernelGGL(gemm_nt_big<Epi>, dim3((unsigned)((g.M / kBigT) * (g.N / kBigT))), dim3(512), 0, st, g, e);
+  else if (g.N % 256 == 0)
+    hipLaunchKernelGGL((gemm_nt<256, Epi>), dim3((unsigned)((g.M / kGT) * (g.N / 256))), dim3(256), 0, st, g, e);
+  else
+    hipLaunchKernelGGL((gemm_nt<128, Epi>), dim3((unsigned)((g.M / kGT) * (g.N / 128))), dim3(256), 0, st, g, e);
+}
 static M2xPlan m2x_plan(const atomic_mamba2_proj_args* a, bool bwd) {
   M2xPlan p;
   p.d = a->heads * a->headdim;
@@ -835,11 +855,24 @@ static M2xPlan m2x_plan(const atomic_mamba2_proj_args* a, bool bwd) {
   p.M = a->batch * a->seqlen;
   p.dm = PlDims{a->batch, a->seqlen, a->heads, 128, p.d, 0.f, (int)a->in_stride};
   // row splits of the weight-gradient GEMM: enough workgroups to fill the chip,
-  // each split a multiple of 64 rows
-  const int tiles = (p.d / kGT) * (p.nt / (p.nt % 256 == 0 ? 256 : 128));
-  int s = 1;
-  while (s * tiles < 1024 && p.M % (2 * s * kGK) == 0) s *= 2;
-  p.splits = s;
+  // each split a multiple of 64 rows (32 in the large tiles)
+  p.dw_big = p.nt % kBigT == 0 && p.M >= 512;
+  if (p.dw_big) {
+    // 256 x 256 tiles, one workgroup per CU: as many splits as fill the 256 CUs
+    // once (a second, part-filled round costs more: eight splits of 42 tiles
+    // 0.265 ms, six 0.206), of at least 128 rows; the last one may be shorter
+    const int tiles = (p.d / kBigT) * (p.nt / kBigT);
+    int s = tiles < 256 ? 256 / tiles : 1;
+    if (s > p.M / 128) s = p.M / 128;
+    p.rows = (p.M / kBigK + s - 1) / s * kBigK;
+    p.splits = (p.M + p.rows - 1) / p.rows;
+  } else {
+    const int tiles = (p.d / kGT) * (p.nt / (p.nt % 256 == 0 ? 256 : 128));
+    int s = 1;
+    while (s * tiles < 1024 && p.M % (2 * s * kGK) == 0) s *= 2;
+    p.splits = s;
+    p.rows = p.M / s;
+  }
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += al(bytes); return o; };
@@ -895,12 +928,7 @@ extern "C" int atomic_mamba2_proj_fwd(const atomic_mamba2_proj_args* a, const vo
   rc = L("m2p_proj_gemm", [&] {
     const GemmNT g{(const bf16*)x_bc, (long long)a->in_stride, wt, (long long)p.d, p.M, p.nt, p.d};
     const M2ProjEpi e{p.d, p.n, b_dt, (bf16*)dt, (bf16*)B, (bf16*)C, (bf16*)dt_pre, (bf16*)b_pre, (bf16*)c_pre};
-    if (p.nt % 256 == 0)
-      hipLaunchKernelGGL((gemm_nt<256, M2ProjEpi>), dim3((unsigned)((p.M / kGT) * (p.nt / 256))), dim3(256), 0, st, g,
-                         e);
-    else
-      hipLaunchKernelGGL((gemm_nt<128, M2ProjEpi>), dim3((unsigned)((p.M / kGT) * (p.nt / 128))), dim3(256), 0, st, g,
-                         e);
+    m2x_gemm_nt(g, e, aligned16({b_dt, dt, B, C, dt_pre, b_pre, c_pre}), st);
   });
   if (rc) return rc;
   return L("m2_prologue_elem_fwd", [&] {  // A only (no element ranges)
@@ -945,7 +973,7 @@ extern "C" int atomic_mamba2_proj_bwd(const atomic_mamba2_proj_args* a, const vo
   });
   if (rc) return rc;
   rc = L("m2p_vjp", [&] {
-    const size_t nth = (size_t)(p.M / 32) * (p.nt / 8);
+    const size_t nth = (size_t)(p.M / 32) * (p.nt / 4);
     hipLaunchKernelGGL(m2p_vjp, dim3((unsigned)((nth + 255) / 256)), dim3(256), 0, st, p.M, p.d, p.n, a->heads,
                        (const bf16*)dt_pre, (const bf16*)b_pre, (const bf16*)c_pre, a_log, (const bf16*)ddt,
                        (const bf16*)dB, (const bf16*)dC, dA, dpre, dbp, da_log);
@@ -960,12 +988,14 @@ extern "C" int atomic_mamba2_proj_bwd(const atomic_mamba2_proj_args* a, const vo
   rc = L("m2p_dx_gemm", [&] {
     const GemmNT g{dpre, (long long)p.nt, w, (long long)p.nt, p.M, p.d, p.nt};
     const M2DxEpi e{dxc, p.d, (bf16*)dx_bc, (long long)a->in_stride};
-    hipLaunchKernelGGL((gemm_nt<256, M2DxEpi>), dim3((unsigned)((p.M / kGT) * (p.d / 256))), dim3(256), 0, st, g, e);
+    m2x_gemm_nt(g, e, aligned16({dx_bc}), st);
   });
   if (rc) return rc;
   rc = L("m2p_dw_gemm", [&] {
-    const GemmTN g{(const bf16*)x_bc, (long long)a->in_stride, dpre, (long long)p.nt, p.d, p.nt, p.M / p.splits, dwp};
-    if (p.nt % 256 == 0)
+    const GemmTN g{(const bf16*)x_bc, (long long)a->in_stride, dpre, (long long)p.nt, p.d, p.nt, p.rows, dwp, p.M};
+    if (p.dw_big)
+      hipLaunchKernelGGL(gemm_tn_big, dim3((unsigned)(p.splits * (p.d / kBigT) * (p.nt / kBigT))), dim3(512), 0, st, g);
+    else if (p.nt % 256 == 0)
       hipLaunchKernelGGL(gemm_tn<256>, dim3((unsigned)(p.splits * (p.d / kGT) * (p.nt / 256))), dim3(256), 0, st, g);
     else
       hipLaunchKernelGGL(gemm_tn<128>, dim3((unsigned)(p.splits * (p.d / kGT) * (p.nt / 128))), dim3(256), 0, st, g);

@@ -108,3 +108,28 @@ def test_unsupported_shapes_are_rejected_before_launch():
     gparams = [t.cuda() for t in params]
     with pytest.raises(_lib.AtomicError, match="unsupported shape"):
         PL.mamba2_proj_forward(in_proj.cuda()[..., :512], *gparams, 4)
+
+
+@pytest.mark.parametrize("B,L,H,P,N", [
+    (1, 512, 4, 128, 128),     # 128-row tiles for the products, the smallest large-tile weight gradient
+    (1, 11264, 8, 64, 128),    # large tiles forward only (132 of them); 40 row splits, the last of 32 rows
+    (3, 5632, 4, 128, 128),    # large tiles in both directions
+    (2, 5632, 4, 128, 64),     # 640 columns: no large tiles at all
+])
+def test_large_tiles_match_oracle_and_the_small_tiles(B, L, H, P, N):
+    """256 x 256 tiles against the oracle, and the forward's rows bit-identical
+    to a call that is too small for them (the reduction runs in the same order)."""
+    banner(f"mamba2 proj prologue large tiles B={B} L={L} H={H} P={P} N={N}")
+    in_proj, params, cots = _inputs(B, L, H, P, N, B + L + N)
+    d = H * P
+    x_bc = in_proj[..., :d]
+    gp = in_proj.cuda()
+    gparams = [t.cuda() for t in params]
+    outs, pres = PL.mamba2_proj_forward(gp[..., :d], *gparams, H, save=True)
+    grads = PL.mamba2_proj_backward(gp[..., :d], *gparams, H, pres, *(c.cuda() for c in cots))
+    torch.cuda.synchronize()
+    _check(OUTS, outs, op.mamba2_proj_prologue(x_bc, *params, H))
+    _check(GRADS, grads, op.mamba2_proj_prologue_grads([x_bc] + params, cots, H))
+    small, small_pres = PL.mamba2_proj_forward(gp[0, :256, :d].clone()[None], *gparams, H, save=True)
+    for name, a, b in zip(OUTS[1:4] + PRES, outs[1:4] + pres, small[1:4] + small_pres):
+        assert torch.equal(a[:1, :256], b), name
