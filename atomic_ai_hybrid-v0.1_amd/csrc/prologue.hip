@@ -42,6 +42,19 @@ struct PlDims {
 };
 
 __device__ __forceinline__ float bfr(float x) { return (float)(bf16)x; }
+// bf16-rounds every element, two to a conversion (three instructions a pair
+// where single roundings take four)
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+template <int N>
+__device__ __forceinline__ void bfr_all(float (&x)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; j += 2) {
+    const bf16x2 v = {(bf16)x[j], (bf16)x[j + 1]};
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    x[j] = __uint_as_float(u << 16);
+    x[j + 1] = __uint_as_float(u & 0xffff0000u);
+  }
+}
 // logistic with the hardware reciprocal (about 1 ulp; every use rounds to bf16)
 __device__ __forceinline__ float sigm(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 // jax.nn.softplus(x) = logaddexp(x, 0) = max(x, 0) + log(1 + e^{-|x|}); the
@@ -68,10 +81,10 @@ __device__ __forceinline__ float clip_g(float v, float c) {
   const float a = fabsf(v);
   return a < c ? 1.f : (a == c ? 0.5f : 0.f);
 }
-// nan_to_num(clip(x, -c, c)) (model.py:615-617)
+// nan_to_num(clip(x, -c, c)) (model.py:615-617), as a select
 __device__ __forceinline__ float sanit(float x, float c) {
-  if (__builtin_isnan(x)) return 0.f;
-  return fminf(fmaxf(x, -c), c);
+  const float y = __builtin_amdgcn_fmed3f(x, -c, c);
+  return __builtin_isnan(x) ? 0.f : y;
 }
 
 // v + v of the lane that the DPP control CTRL selects (within a 16-lane row)
@@ -118,9 +131,27 @@ __device__ __forceinline__ void conv_silu(const ConvW<CPL>& W, const float (&win
     float acc = 0.f;
 #pragma unroll
     for (int tp = 0; tp < kDc; ++tp) acc += win[tp][j] * W.w[tp][j];
-    pre[j] = bfr(bfr(acc) + W.b[j]);
-    s[j] = bfr(pre[j] * sigm(pre[j]));
+    pre[j] = acc;
   }
+  bfr_all(pre);
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) pre[j] += W.b[j];
+  bfr_all(pre);
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) s[j] = pre[j] * sigm(pre[j]);
+  bfr_all(s);
+}
+
+// the sum of a head's bf16-rounded squares, rounded
+template <int G, int CPL>
+__device__ __forceinline__ float head_squares(const float (&s)[CPL]) {
+  float q[CPL], ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) q[j] = s[j] * s[j];
+  bfr_all(q);
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) ss += q[j];
+  return bfr(head_sum<G>(ss));
 }
 
 // ---------------------------------------------------------------- forward
@@ -129,10 +160,9 @@ __device__ __forceinline__ void conv_silu(const ConvW<CPL>& W, const float (&win
 enum { kNorm = 0, kClip50 = 1, kPlain = 2 };
 
 template <int MODE, int DH>
-__global__ __launch_bounds__(256) void prologue_conv_fwd(PlDims dm, const bf16* __restrict__ lin,
-                                                         const float* __restrict__ conv_w,
-                                                         const float* __restrict__ conv_b,
-                                                         bf16* __restrict__ out) {
+__device__ __forceinline__ void conv_fwd_tile(const PlDims& dm, const bf16* __restrict__ lin,
+                                              const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+                                              bf16* __restrict__ out) {
   constexpr int G = DH / 8;
   const int lane = lane_id();
   const int nblk = dm.d / 512, ntile = dm.L / kTileF;
@@ -164,13 +194,10 @@ __global__ __launch_bounds__(256) void prologue_conv_fwd(PlDims dm, const bf16* 
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = sanit(s[j], 1e3f);
     } else {
-      float ss = 0.f;
+      const float r = bfr(rsqrtf(bfr(head_squares<G>(s) + dm.eps * dm.eps)));
+      // rounded by the store: the clip's bounds are bf16 values
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss += bfr(s[j] * s[j]);
-      ss = bfr(head_sum<G>(ss));
-      const float r = bfr(rsqrtf(bfr(ss + dm.eps * dm.eps)));
-#pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] = sanit(bfr(s[j] * r), 1e3f);
+      for (int j = 0; j < 8; ++j) y[j] = sanit(s[j] * r, 1e3f);
     }
     store8(o + (size_t)t * dm.d, y);
 #pragma unroll
@@ -178,6 +205,30 @@ __global__ __launch_bounds__(256) void prologue_conv_fwd(PlDims dm, const bf16* 
 #pragma unroll
       for (int j = 0; j < 8; ++j) win[tp][j] = win[tp + 1][j];
   }
+}
+
+template <int MODE, int DH>
+__global__ __launch_bounds__(256) void prologue_conv_fwd(PlDims dm, const bf16* __restrict__ lin,
+                                                         const float* __restrict__ conv_w,
+                                                         const float* __restrict__ conv_b,
+                                                         bf16* __restrict__ out) {
+  conv_fwd_tile<MODE, DH>(dm, lin, conv_w, conv_b, out);
+}
+
+// The GDN2 block's three convolutions in one launch (blockIdx.y = q, k, v).
+// Alone, each launch's waves are all resident at once and load, compute and
+// store in step with one another; together, one convolution's loads and
+// stores run under another's arithmetic (with the backward's merged launch the
+// prologue's forward + backward at B4 T4096 H16 D128: 576 -> 537 us).
+struct Conv3F { const bf16* lin[3]; bf16* out[3]; };
+template <int DH>
+__global__ __launch_bounds__(256) void prologue_conv3_fwd(PlDims dm, Conv3F p, const float* __restrict__ conv_w,
+                                                          const float* __restrict__ conv_b) {
+  const int i = blockIdx.y;
+  const float* w = conv_w + (size_t)i * dm.d * kDc;
+  const float* b = conv_b + (size_t)i * dm.d;
+  if (i < 2) conv_fwd_tile<kNorm, DH>(dm, i ? p.lin[1] : p.lin[0], w, b, i ? p.out[1] : p.out[0]);
+  else conv_fwd_tile<kClip50, DH>(dm, p.lin[2], w, b, p.out[2]);
 }
 
 // b, w = sigmoid(pre); g = nan_to_num(-exp(clip(a)) softplus(f)); 8 channels per thread
@@ -221,24 +272,23 @@ __device__ __forceinline__ void conv_out_vjp(const ConvW<CPL>& W, const float (&
   if (MODE == kClip50) {
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
-      const float v = fminf(fmaxf(s[j], -50.f), 50.f);
-      ds[j] = bfr(dy[j] * clip_g(v, 1e3f) * clip_g(s[j], 50.f));
+      // the output clip passes everything within +-50
+      ds[j] = dy[j] * clip_g(s[j], 50.f);
     }
   } else if (MODE == kPlain) {
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) ds[j] = bfr(dy[j] * clip_g(s[j], 1e3f));
+    for (int j = 0; j < CPL; ++j) ds[j] = dy[j] * clip_g(s[j], 1e3f);
   } else {
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) ss += bfr(s[j] * s[j]);
-    ss = bfr(head_sum<G>(ss));
+    const float ss = head_squares<G>(s);
     const float r = bfr(rsqrtf(bfr(ss + eps * eps)));
     // output clip (|y| <= 1 passes), then the gradient sanitiser (model.py:206-214)
-    float gy[CPL], dot = 0.f;
+    float gy[CPL], y[CPL], dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) y[j] = s[j] * r;
+    bfr_all(y);
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
-      const float y = bfr(s[j] * r);
-      float g = dy[j] * clip_g(y, 1e3f);
+      float g = dy[j] * clip_g(y[j], 1e3f);
       g = __builtin_isnan(g) ? 0.f : fminf(fmaxf(g, -1e3f), 1e3f);
       gy[j] = g;
       dot += g * s[j];
@@ -246,13 +296,15 @@ __device__ __forceinline__ void conv_out_vjp(const ConvW<CPL>& W, const float (&
     dot = head_sum<G>(dot);
     const float r3 = r * r * r;
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) ds[j] = bfr(gy[j] * r - s[j] * r3 * dot);
+    for (int j = 0; j < CPL; ++j) ds[j] = gy[j] * r - s[j] * r3 * dot;
   }
+  bfr_all(ds);
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const float sg = sigm(pre[j]);
-    e[j] = bfr(ds[j] * (sg * (1.f + pre[j] * (1.f - sg))));
+    e[j] = ds[j] * (sg * (1.f + pre[j] * (1.f - sg)));
   }
+  bfr_all(e);
 }
 
 // 4 bf16 of a row as floats, from a raw 8-byte piece
@@ -303,9 +355,10 @@ __device__ __forceinline__ void combine_partials(float (&v)[NV][CPL], float* __r
 // partial row index = (batch, tile group).
 constexpr int kCplB = 4;
 template <int MODE, int DH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void prologue_conv_bwd(
-    PlDims dm, const bf16* __restrict__ lin, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
-    const bf16* __restrict__ dout, bf16* __restrict__ dlin, float* __restrict__ part) {
+__device__ __forceinline__ void conv_bwd_tile(const PlDims& dm, const bf16* __restrict__ lin,
+                                              const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+                                              const bf16* __restrict__ dout, bf16* __restrict__ dlin,
+                                              float* __restrict__ part) {
   constexpr int CPL = kCplB, G = DH / CPL, NV = kDc + 1;  // partials: the 4 taps, then the bias
   const int lane = lane_id();
   const int nblk = dm.d / (64 * CPL), ngrp = dm.L / (4 * kTileB);
@@ -370,7 +423,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   combine_partials<NV, CPL>(acc, part + ((size_t)b * ngrp + grp) * dm.d * NV, c);
 }
 
-// b, w, g gradients; per-head partial sums of da
+template <int MODE, int DH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void prologue_conv_bwd(
+    PlDims dm, const bf16* __restrict__ lin, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+    const bf16* __restrict__ dout, bf16* __restrict__ dlin, float* __restrict__ part) {
+  conv_bwd_tile<MODE, DH>(dm, lin, conv_w, conv_b, dout, dlin, part);
+}
+
+// The three convolutions of the GDN2 block in one launch, as in the forward.
+struct Conv3B { const bf16* lin[3]; const bf16* dout[3]; bf16* dlin[3]; };
+template <int DH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void prologue_conv3_bwd(
+    PlDims dm, Conv3B p, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+    float* __restrict__ part, size_t part_n) {
+  const int i = blockIdx.y;
+  const float* w = conv_w + (size_t)i * dm.d * kDc;
+  const float* b = conv_b + (size_t)i * dm.d;
+  float* pt = part + i * part_n;
+  if (i < 2)
+    conv_bwd_tile<kNorm, DH>(dm, i ? p.lin[1] : p.lin[0], w, b, i ? p.dout[1] : p.dout[0],
+                             i ? p.dlin[1] : p.dlin[0], pt);
+  else
+    conv_bwd_tile<kClip50, DH>(dm, p.lin[2], w, b, p.dout[2], p.dlin[2], pt);
+}
+
+// b, w, g gradients; per-head partial sums of da.  A workgroup's four waves take
+// eight tokens each of one 32-token tile: with a tile to a wave the launch
+// left two waves per SIMD, too few loads in flight (B4 T4096 H16 D128: 170 ->
+// 128 us, 3.9 -> 5.2 TB/s).
 template <int DH>
 __global__ __launch_bounds__(256) void prologue_gates_bwd(PlDims dm, const bf16* __restrict__ b_pre,
                                                           const bf16* __restrict__ w_pre,
@@ -380,19 +460,18 @@ __global__ __launch_bounds__(256) void prologue_gates_bwd(PlDims dm, const bf16*
                                                           const float* __restrict__ dg, bf16* __restrict__ dbp,
                                                           bf16* __restrict__ dwp, bf16* __restrict__ dfp,
                                                           float* __restrict__ part_a) {
-  constexpr int G = DH / 8;
-  const int lane = lane_id();
+  constexpr int G = DH / 8, HB = 512 / DH;
+  __shared__ float red[4][HB];
+  const int lane = lane_id(), w = wave_id();
   const int nblk = dm.d / 512, ntile = dm.L / kTileB;
-  const int wv = blockIdx.x * 4 + wave_id();
-  if (wv >= dm.B * ntile * nblk) return;  // wave-uniform
-  const int cb = wv % nblk, tile = (wv / nblk) % ntile, b = wv / (nblk * ntile);
+  const int cb = blockIdx.x % nblk, tile = (blockIdx.x / nblk) % ntile, b = blockIdx.x / (nblk * ntile);
   const int c = cb * 512 + 8 * lane, h = c / DH;
   const float araw = a_param[h];
   const float ea = __expf(fminf(fmaxf(araw, -20.f), 20.f)), ga = clip_g(araw, 20.f);
   float da = 0.f;
-#pragma unroll 4
-  for (int t = tile * kTileB; t < (tile + 1) * kTileB; ++t) {
-    const size_t e = ((size_t)b * dm.L + t) * dm.d + c;
+#pragma unroll 2
+  for (int i = 0; i < kTileB / 4; ++i) {
+    const size_t e = ((size_t)b * dm.L + tile * kTileB + w * (kTileB / 4) + i) * dm.d + c;
     float bv[8], wv8[8], fv[8], gb[8], gw[8], gg[8], o1[8], o2[8], o3[8];
     load8(b_pre + e, bv);
     load8(w_pre + e, wv8);
@@ -417,8 +496,12 @@ __global__ __launch_bounds__(256) void prologue_gates_bwd(PlDims dm, const bf16*
     store8(dfp + e, o3);
   }
   da = head_sum<G>(da);
-  // one partial per (wave, head of the block): lane 0 of each head group writes
-  if ((lane % G) == 0) part_a[(size_t)wv * (512 / DH) + lane / G] = da;
+  // one partial per (tile, head of the block)
+  if ((lane % G) == 0) red[w][lane / G] = da;
+  __syncthreads();
+  if (threadIdx.x < HB)
+    part_a[(size_t)blockIdx.x * HB + threadIdx.x] =
+        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
 }
 
 // Column sums of the partial rows: out[c] = sum_r part[r][c] for c < ncol
@@ -622,13 +705,8 @@ extern "C" int atomic_gdn2_prologue_fwd(const atomic_gdn2_prologue_args* a, cons
   auto run = [&](auto Dc) {
     constexpr int DH = decltype(Dc)::value;
     int r = L("prologue_conv_fwd", [&] {
-      const size_t ow = (size_t)dm.d * kDc, ob = (size_t)dm.d;
-      hipLaunchKernelGGL((prologue_conv_fwd<kNorm, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[0], conv_w,
-                         conv_b, outs[0]);
-      hipLaunchKernelGGL((prologue_conv_fwd<kNorm, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[1],
-                         conv_w + ow, conv_b + ob, outs[1]);
-      hipLaunchKernelGGL((prologue_conv_fwd<kClip50, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[2],
-                         conv_w + 2 * ow, conv_b + 2 * ob, outs[2]);
+      const Conv3F p = {{lins[0], lins[1], lins[2]}, {outs[0], outs[1], outs[2]}};
+      hipLaunchKernelGGL(prologue_conv3_fwd<DH>, dim3(nconv, 3), dim3(256), 0, st, dm, p, conv_w, conv_b);
     });
     if (r) return r;
     return L("prologue_gates_fwd", [&] {
@@ -666,21 +744,16 @@ extern "C" int atomic_gdn2_prologue_bwd(const atomic_gdn2_prologue_args* a, cons
   Launch L{a->profile, st};
   const int ngrp = dm.L / (4 * kTileB);
   const unsigned nconv = (unsigned)((size_t)dm.B * ngrp * (dm.d / (64 * kCplB)));
-  const unsigned ngate = (unsigned)(((size_t)dm.B * (dm.L / kTileB) * (dm.d / 512) + 3) / 4);
+  const unsigned ngate = (unsigned)((size_t)dm.B * (dm.L / kTileB) * (dm.d / 512));
   const bf16* lins[3] = {(const bf16*)q_lin, (const bf16*)k_lin, (const bf16*)v_lin};
   const bf16* dys[3] = {(const bf16*)dq, (const bf16*)dk, (const bf16*)dv};
   bf16* dls[3] = {(bf16*)dq_lin, (bf16*)dk_lin, (bf16*)dv_lin};
   auto run = [&](auto Dc) {
     constexpr int DH = decltype(Dc)::value;
     int r = L("prologue_conv_bwd", [&] {
-      const size_t ow = (size_t)dm.d * kDc, ob = (size_t)dm.d;
       const size_t op = (size_t)dm.B * ngrp * dm.d * (kDc + 1);  // one conv's partial rows
-      hipLaunchKernelGGL((prologue_conv_bwd<kNorm, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[0], conv_w,
-                         conv_b, dys[0], dls[0], pconv);
-      hipLaunchKernelGGL((prologue_conv_bwd<kNorm, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[1],
-                         conv_w + ow, conv_b + ob, dys[1], dls[1], pconv + op);
-      hipLaunchKernelGGL((prologue_conv_bwd<kClip50, DH>), dim3(nconv), dim3(256), 0, st, dm, lins[2],
-                         conv_w + 2 * ow, conv_b + 2 * ob, dys[2], dls[2], pconv + 2 * op);
+      const Conv3B p = {{lins[0], lins[1], lins[2]}, {dys[0], dys[1], dys[2]}, {dls[0], dls[1], dls[2]}};
+      hipLaunchKernelGGL(prologue_conv3_bwd<DH>, dim3(nconv, 3), dim3(256), 0, st, dm, p, conv_w, conv_b, pconv, op);
     });
     if (r) return r;
     return L("prologue_gates_bwd", [&] {
