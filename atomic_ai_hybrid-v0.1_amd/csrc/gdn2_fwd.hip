@@ -129,8 +129,8 @@ struct IntraLds {
   static constexpr int off_x = off_af + AF;                 // fp32 inverse
   static constexpr int end_a = off_x + AF;
   static constexpr int off_tot = (end_ops > end_a ? end_ops : end_a);
-  // cumsum totals of the waves; then the solve's products: two 16-row ones, one 32-row one
-  static constexpr int LT = 36, S16 = 16 * 17 * 4, SOLVE = 2 * S16 + 32 * LT * 4;
+  // cumsum totals of the waves; then the solve's products, one a wave
+  static constexpr int S16 = 16 * 17 * 4, SOLVE = (C / 16 - 1) * S16;
   static constexpr int TOT = NW * K * 4 > SOLVE ? NW * K * 4 : SOLVE;
   static constexpr int off_gl = off_tot + TOT;
   static constexpr int off_flag = off_gl + K * 4;
@@ -187,10 +187,9 @@ enum { kIntraAll = 0, kIntraScores = 1, kIntraSolve = 2, kIntraRecompute = 3 };
 
 //
 // One chunk is a chain of short phases (loads and cumsum, element-wise operands,
-// scores, four 16-row substitutions, their 32- and 64-row combination, the two
-// products), so the kernel is latency, hidden by eight waves per workgroup and
-// two workgroups per CU: with four waves and a column of blocks per wave in the
-// solve, one chunk took 30k cycles (14.8 us at B1 T64 H8 K = 128, 0.383 ms at B4
+// scores, four 16-row substitutions, the blocks below them column by column, the
+// two products), so the kernel is latency, hidden by eight waves per workgroup and
+// two workgroups per CU: with four waves one chunk took 30k cycles (14.8 us at B1 T64 H8 K = 128, 0.383 ms at B4
 // T8192 H16), so 12.4 us and 0.330 ms, the latter 4.8 TB/s of what the kernel
 // has to move and as fast as a large copy.
 template <typename T, int C, int K, int V, int ST = kIntraAll>
@@ -416,7 +415,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   const T* opA;
   int ldA;
   if constexpr (ST != kIntraRecompute) {
-  static_assert(C == 64 && NW >= 4, "two levels of 2 x 2 blocks over 16-row blocks");
+  static_assert(NB <= NW, "a 16-row block per wave");
   // Diagonal 16x16 blocks by forward substitution (wave w, lane = column).
   {
     const int lane = lane_id();
@@ -440,34 +439,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     }
   }
   __syncthreads();
-  // [[A0, 0], [-A1 T A0, A1]] of two 16-row blocks for both 32-row halves
-  if (wv_id < 2) {
-    const int o = 32 * wv_id;
+  // Off-diagonal blocks, one column block per wave (no wave reads another's column):
+  //   A_mn = -A_mm (sum_{k=n}^{m-1} T_mk A_kn)
+  if (wv_id < NB - 1) {
+    const int nb = wv_id;
     float* scr = sTot + wv_id * (L::S16 / 4);  // private to this wave
-    const f32x4 p = tile_mma<float, false, true>(zero4(), sAf + o, L::LA, sX + o * L::LA + o, L::LA, o + 16, 0, 16);
-    store_tile_n(scr, 17, 0, 0, p);
-    wave_lds_sync();
-    f32x4 a = tile_mma<float, false, true>(zero4(), sX + (o + 16) * L::LA + o + 16, L::LA, scr, 17, 0, 0, 16);
+    for (int mb = nb + 1; mb < NB; ++mb) {
+      const f32x4 p = tile_mma<float, false, true>(zero4(), sAf + 16 * nb, L::LA, sX + 16 * nb * L::LA, L::LA, 16 * mb,
+                                                   16 * nb, 16 * (mb - nb));
+      store_tile_n(scr, 17, 0, 0, p);
+      wave_lds_sync();
+      f32x4 a = tile_mma<float, false, true>(zero4(), sX + 16 * mb * L::LA + 16 * mb, L::LA, scr, 17, 0, 0, 16);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = -a[i];
-    store_tile_n(sX, L::LA, o + 16, o, a);
-  }
-  __syncthreads();
-  // the same of the two halves: a 16 x 16 tile (m, n) per wave, over the nonzero blocks
-  float* s32 = sTot + 2 * (L::S16 / 4);
-  const int tm = (wv_id >> 1) & 1, tn = wv_id & 1;
-  if (wv_id < 4) {
-    const f32x4 p = tile_mma<float, false, true>(zero4(), sAf + 16 * tn, L::LA, sX + 16 * tn * L::LA, L::LA,
-                                                 32 + 16 * tm, 16 * tn, 32 - 16 * tn);
-    store_tile_n(s32, L::LT, 16 * tm, 16 * tn, p);
-  }
-  __syncthreads();
-  if (wv_id < 4) {
-    f32x4 a = tile_mma<float, false, true>(zero4(), sX + 32 * L::LA + 32, L::LA, s32, L::LT, 16 * tm, 16 * tn,
-                                           16 + 16 * tm);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = -a[i];
-    store_tile_n(sX, L::LA, 32 + 16 * tm, 16 * tn, a);
+      for (int i = 0; i < 4; ++i) a[i] = -a[i];
+      store_tile_n(sX, L::LA, 16 * mb, 16 * nb, a);
+      wave_lds_sync();  // the next row block reads this one
+    }
   }
   __syncthreads();
   // n2n, operand-type copy, global A

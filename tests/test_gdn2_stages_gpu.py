@@ -123,6 +123,47 @@ def test_kernels_a_b_c_chained_equal_the_one_pass_build_in_fp32():
         assert torch.equal(x, y), name
 
 
+def _fma(a, b, c):
+    """a b + c, rounded to float32 once (the product is exact in float64)."""
+    return (a.double() * b.double() + c.double()).float()
+
+
+def _solve_in_order(akk):
+    """(I + akk)^-1 in float32 with the kernels' order of operations: 16-row
+    substitutions, then a column of blocks at a time, every sum one serial chain."""
+    eye = torch.eye(16).expand(*akk.shape[:-2], 16, 16)
+
+    def product(a, b):
+        acc = torch.zeros(*a.shape[:-1], b.shape[-1])
+        for k in range(a.shape[-1]):
+            acc = _fma(a[..., :, k:k + 1], b[..., k:k + 1, :], acc)
+        return acc
+    out = torch.zeros_like(akk)
+    blk = [slice(16 * i, 16 * i + 16) for i in range(4)]
+    for i in range(4):
+        rows, a = list(eye.unbind(-2)), akk[..., blk[i], blk[i]]
+        for j in range(16):
+            for r in range(j + 1, 16):
+                rows[r] = _fma(-a[..., r, j:j + 1], rows[j], rows[r])
+        out[..., blk[i], blk[i]] = torch.stack(rows, -2)
+    for n in range(4):
+        for m in range(n + 1, 4):
+            s = product(akk[..., blk[m], 16 * n:16 * m], out[..., 16 * n:16 * m, blk[n]])
+            out[..., blk[m], blk[n]] = -product(out[..., blk[m], blk[m]], s)
+    return out
+
+
+def test_solve_keeps_its_order_of_sums():
+    """The 64-row inverse is formed in one stated order, whatever the number of
+    threads: another order is as accurate, but flips bf16 roundings of
+    w_pseudo and u, and with them bits of every output and gradient."""
+    banner("gdn2 solve order of sums")
+    Akk = torch.tril(torch.randn(2, 3, 4, 64, 64, generator=torch.Generator().manual_seed(64)) / 8.0, -1)
+    A = KB.wy_solve_pallas(Akk.cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(A.cpu(), _solve_in_order(Akk))
+
+
 def test_kernel_c_clips_like_the_reference():
     """Kernel C alone clips w_pseudo and u to +-1e4 (kernel_c_recompute.py:74-78):
     a large A drives them past it."""
