@@ -28,22 +28,34 @@ constexpr float kFactorLimit = 64.f;
 
 // ------------------------------------------------------------------ cumsum
 // Thread map for [C][K] fp32 element-wise passes: column group cg (8
-// columns), segment seg (RS consecutive rows).
+// columns), segment seg (RS consecutive rows).  Whatever the number of
+// threads, a wave covers a quarter of the rows: with 256 threads all columns of
+// them, with 512 half of the columns in segments of half the length.
 template <int C, int K, int NTH = 256>
 struct ColMap {
   static constexpr int NCG = K / 8, NSEG = NTH / NCG, RS = C / NSEG;
+  static constexpr int U = NTH / 256, WCG = NCG / U;  // column groups of a wave
   static_assert(RS >= 1, "chunk too small for the thread mapping");
+  static __device__ __forceinline__ int cg() {
+    return U == 1 ? lane_id() % NCG : (wave_id() & 1) * WCG + lane_id() % WCG;
+  }
+  static __device__ __forceinline__ int seg() {
+    return (U == 1 ? wave_id() : wave_id() >> 1) * (64 / WCG) + lane_id() / WCG;
+  }
 };
 
 // Exclusive scan over the row segments of a ColMap pass: t holds this
 // thread's segment total for its 8 columns; out gets the sum over the lower
 // segments (REV = false) or the higher ones (REV = true).  Within a wave by
-// lane shuffles, across the NW waves through sW (NW * K floats).
-template <int NCG, bool REV, int NW = 4>
+// lane shuffles, across the four waves of a column through sW (4 * K floats).
+// With U > 1, U consecutive segments count as one (t is its total in each).
+template <int NCG, bool REV, int U = 1>
 __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], float* sW) {
-  constexpr int SPW = 64 / NCG;  // segments per wave
-  static_assert(SPW * NCG == 64, "column groups must tile a wave");
-  const int lane = lane_id(), w = wave_id(), sl = lane / NCG, cg = lane % NCG;
+  constexpr int UL = NCG;           // lanes of a segment, or of the U that count as one
+  constexpr int SPW = 64 / UL;      // segments per wave
+  static_assert(SPW * UL == 64, "column groups must tile a wave");
+  const int lane = lane_id(), w = U == 1 ? wave_id() : wave_id() >> 1, sl = lane / UL;
+  const int cg = U == 1 ? lane % NCG : (wave_id() & 1) * (NCG / U) + lane % (NCG / U);
   float x[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) x[j] = t[j];
@@ -51,7 +63,7 @@ __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], 
   for (int d = 1; d < SPW; d <<= 1) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float y = REV ? __shfl_down(x[j], d * NCG) : __shfl_up(x[j], d * NCG);
+      const float y = REV ? __shfl_down(x[j], d * UL) : __shfl_up(x[j], d * UL);
       if (REV ? (sl + d < SPW) : (sl >= d)) x[j] += y;
     }
   }
@@ -63,24 +75,33 @@ __device__ __forceinline__ void seg_scan8(const float (&t)[8], float (&out)[8], 
 #pragma unroll
   for (int j = 0; j < 8; ++j) out[j] = x[j] - t[j];
 #pragma unroll
-  for (int w2 = 0; w2 < NW; ++w2)
+  for (int w2 = 0; w2 < 4; ++w2)
     if (REV ? w2 > w : w2 < w) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) out[j] += sW[w2 * NCG * 8 + cg * 8 + j];
     }
 }
 
+// x of the lane that the DPP control CTRL selects (within a 16-lane row)
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
 // gc = cumsum(g) over one chunk (gdn2_wy_reference.py:63) for this thread's
-// RS rows x 8 columns.  Writes gc_last to sGl[K] (sTot: NTH / 64 * K floats of
+// RS rows x 8 columns.  Writes gc_last to sGl[K] (sTot: 4 K floats of
 // scratch).  Returns, uniformly over the workgroup, whether the factorised
 // pairwise decay is unsafe for this chunk: some g > 0, or gc_last below
-// -kFactorLimit in some column.
+// -kFactorLimit in some column.  The order of the additions does not depend on
+// NTH: with 512 threads two lanes continue one serial sum, so that the
+// exponentials, and every bf16 operand rounded from them, are the same bits.
 template <int C, int K, int NTH = 256>
 __device__ __forceinline__ bool chunk_cumsum(const float* __restrict__ g, size_t rs,
                                              float (&gcr)[ColMap<C, K, NTH>::RS][8], float* sTot,
                                              float* sGl) {
   typedef ColMap<C, K, NTH> M;
-  const int tid = threadIdx.x, cg = tid % M::NCG, seg = tid / M::NCG;
+  static_assert(M::U == 1 || (M::U == 2 && 16 % (2 * M::WCG) == 0), "one lane a serial sum, or two of a 16-lane row");
+  const int cg = M::cg(), seg = M::seg();
   bool positive = false;
 #pragma unroll
   for (int rr = 0; rr < M::RS; ++rr) {
@@ -88,12 +109,30 @@ __device__ __forceinline__ bool chunk_cumsum(const float* __restrict__ g, size_t
 #pragma unroll
     for (int j = 0; j < 8; ++j) positive |= gcr[rr][j] > 0.f;
   }
+  if constexpr (M::U == 2) {  // an odd segment goes on from the sum of the even one before it
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float s = gcr[0][j];
+#pragma unroll
+      for (int rr = 1; rr < M::RS; ++rr) s += gcr[rr][j];
+      s = dpp_mov<0x110 + M::WCG>(s);  // row_shr
+      if (seg & 1) gcr[0][j] += s;
+    }
+  }
 #pragma unroll
   for (int rr = 1; rr < M::RS; ++rr)
 #pragma unroll
     for (int j = 0; j < 8; ++j) gcr[rr][j] += gcr[rr - 1][j];
-  float off[8];
-  seg_scan8<M::NCG, false, NTH / 64>(gcr[M::RS - 1], off, sTot);
+  float tot[8], off[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    tot[j] = gcr[M::RS - 1][j];
+    if constexpr (M::U == 2) {
+      const float s = dpp_mov<0x100 + M::WCG>(tot[j]);  // row_shl
+      if (!(seg & 1)) tot[j] = s;
+    }
+  }
+  seg_scan8<M::NCG, false, M::U>(tot, off, sTot);
 #pragma unroll
   for (int rr = 0; rr < M::RS; ++rr)
 #pragma unroll
@@ -129,9 +168,9 @@ struct IntraLds {
   static constexpr int off_x = off_af + AF;                 // fp32 inverse
   static constexpr int end_a = off_x + AF;
   static constexpr int off_tot = (end_ops > end_a ? end_ops : end_a);
-  // cumsum totals of the waves; then the solve's products, one a wave
+  // cumsum totals of the row quarters; then the solve's products, one a wave
   static constexpr int S16 = 16 * 17 * 4, SOLVE = (C / 16 - 1) * S16;
-  static constexpr int TOT = NW * K * 4 > SOLVE ? NW * K * 4 : SOLVE;
+  static constexpr int TOT = 4 * K * 4 > SOLVE ? 4 * K * 4 : SOLVE;
   static constexpr int off_gl = off_tot + TOT;
   static constexpr int off_flag = off_gl + K * 4;
   static constexpr int total = off_flag + 16;
@@ -189,9 +228,12 @@ enum { kIntraAll = 0, kIntraScores = 1, kIntraSolve = 2, kIntraRecompute = 3 };
 // One chunk is a chain of short phases (loads and cumsum, element-wise operands,
 // scores, four 16-row substitutions, the blocks below them column by column, the
 // two products), so the kernel is latency, hidden by eight waves per workgroup and
-// two workgroups per CU: with four waves one chunk took 30k cycles (14.8 us at B1 T64 H8 K = 128, 0.383 ms at B4
-// T8192 H16), so 12.4 us and 0.330 ms, the latter 4.8 TB/s of what the kernel
-// has to move and as fast as a large copy.
+// two workgroups per CU: with four waves one chunk took 17.8 us at B1 T64 H8 K =
+// 128 and the kernel 0.367 ms at B4 T8192 H16, so 11.9 us and 0.316 ms, the latter
+// 5.0 TB/s of what the kernel has to move and as fast as a large copy.  The
+// inverse in two levels of 2 x 2 blocks, and a cumsum whose waves take whole
+// rows (0.312 ms), were as fast or faster but add in another order, which
+// moved the bf16 gradients by 8e-4 of themselves.
 template <typename T, int C, int K, int V, int ST = kIntraAll>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 4 : 2, 4))) void gdn2_fwd_intra(Gdn2Dims dm, const T* __restrict__ q,
                                                      const T* __restrict__ k, const T* __restrict__ v,
@@ -225,7 +267,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   const T* wc = w + t0 * dm.rw + (size_t)h * V;
 
   // q, k, b, v, w are requested before the cumsum of g, so their latency overlaps it
-  const int cg = tid % L::NCG, seg = tid / L::NCG;
+  typedef ColMap<C, K, L::NTH> M;
+  const int cg = M::cg(), seg = M::seg();
   const int cgv = tid % L::NCGV, segv = tid / L::NCGV;
   constexpr bool kRows = ST != kIntraSolve;                          // reads q, k, b, g
   constexpr bool kVals = ST == kIntraAll || ST == kIntraRecompute;   // reads v, w; writes qg, kg

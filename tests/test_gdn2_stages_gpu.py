@@ -164,6 +164,39 @@ def test_solve_keeps_its_order_of_sums():
     assert torch.equal(A.cpu(), _solve_in_order(Akk))
 
 
+def _scan_last(g):
+    """The last row of the kernels' cumsum of g [..., 64, K] float32: serial sums
+    of K / 32 rows, doubling scans over a quarter of the chunk, then the
+    quarters in turn."""
+    K = g.shape[-1]
+    rs = K // 32
+    t = g.reshape(*g.shape[:-2], 4, 16 // rs, rs, K)
+    tot = t[..., 0, :]
+    for i in range(1, rs):
+        tot = tot + t[..., i, :]
+    x, d, n = tot, 1, 16 // rs
+    while d < n:
+        x = torch.cat([x[..., :d, :], x[..., d:, :] + x[..., :-d, :]], -2)
+        d *= 2
+    off = x[..., 3, -1, :] - tot[..., 3, -1, :]
+    for q in range(3):
+        off = off + x[..., q, -1, :]
+    return tot[..., 3, -1, :] + off
+
+
+@pytest.mark.parametrize("dtype,K", [(F32, 64), (F32, 128), (BF16, 64), (BF16, 128)])
+def test_cumsum_keeps_its_order_of_sums(dtype, K):
+    """The gates' cumsum is formed in one stated order, whatever the number of
+    threads (see the solve's test): qg, kg and the scores are exponentials of it."""
+    B, T, H = 2, 256, 3
+    banner(f"gdn2 cumsum order of sums {dtype} K{K}")
+    q, k, v, w, b, g = _inputs(B, T, H, K, dtype, 83 + K)
+    gc_last = KD.build_chunk_wy(*(t.cuda() for t in (q, k, v, w, b, g)), 0.9)[6]
+    torch.cuda.synchronize()
+    gc = g.float().reshape(B, T // 64, 64, H, K).permute(0, 3, 1, 2, 4)
+    assert torch.equal(gc_last.cpu(), _scan_last(gc))
+
+
 def test_kernel_c_clips_like_the_reference():
     """Kernel C alone clips w_pseudo and u to +-1e4 (kernel_c_recompute.py:74-78):
     a large A drives them past it."""
