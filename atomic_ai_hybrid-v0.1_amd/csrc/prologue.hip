@@ -895,12 +895,13 @@ static int m2x_check(const atomic_mamba2_proj_args* a) {
 
 // Workspace: the packed bf16 weights [W_dt | W_B | W_C] (either layout); for
 // the backward also dPre [M][d + 2n] bf16, the convolution path's dx [M][d]
-// bf16, the weight-gradient partials [splits][d][d + 2n] fp32, the b_dt
+// bf16, the weight-gradient partials [splits][d][d + 2n] fp32 (of the GEMM with more splits), the b_dt
 // partials [M / 32][d] and sums [d] fp32, and the convolution's partial rows.
+struct M2xSplit { int n, rows; };  // row splits of the weight-gradient GEMM, rows of one
 struct M2xPlan {
   PlDims dm;
-  int M, d, n, nt, splits, rows;
-  bool dw_big;
+  int M, d, n, nt;
+  M2xSplit dw, dw_big;  // gemm_tn's, gemm_tn_big's (n = 0: not for these sizes)
   size_t o_w, o_dpre, o_dxc, o_dw, o_dbp, o_dbs, o_conv, o_convsum, total;
 };
 static bool aligned16(std::initializer_list<const void*> ps) {
@@ -910,10 +911,11 @@ static bool aligned16(std::initializer_list<const void*> ps) {
 }
 // C = A Bt^T over rows: 256 x 256 tiles where both sides divide and there are
 // more than 128 of them (with fewer, twice as many workgroups of 128 x 256
-// leave less of the chip idle) and the outputs take 16-byte stores.
+// leave less of the chip idle), the outputs take 16-byte stores and the operands
+// 16-byte loads to LDS (gemm_nt loads to registers, from any address).
 template <typename Epi>
 static void m2x_gemm_nt(const GemmNT& g, const Epi& e, bool aligned, hipStream_t st) {
-  if (aligned && g.M % kBigT == 0 && g.N % kBigT == 0 && (g.M / kBigT) * (g.N / kBigT) > 128)
+  if (aligned && aligned16({g.A, g.Bt}) && g.M % kBigT == 0 && g.N % kBigT == 0 && (g.M / kBigT) * (g.N / kBigT) > 128)
     hipLaunchKernelGGL(gemm_nt_big<Epi>, dim3((unsigned)((g.M / kBigT) * (g.N / kBigT))), dim3(512), 0, st, g, e);
   else if (g.N % 256 == 0)
     hipLaunchKernelGGL((gemm_nt<256, Epi>), dim3((unsigned)((g.M / kGT) * (g.N / 256))), dim3(256), 0, st, g, e);
@@ -927,24 +929,21 @@ static M2xPlan m2x_plan(const atomic_mamba2_proj_args* a, bool bwd) {
   p.nt = p.d + 2 * p.n;
   p.M = a->batch * a->seqlen;
   p.dm = PlDims{a->batch, a->seqlen, a->heads, 128, p.d, 0.f, (int)a->in_stride};
-  // row splits of the weight-gradient GEMM: enough workgroups to fill the chip,
-  // each split a multiple of 64 rows (32 in the large tiles)
-  p.dw_big = p.nt % kBigT == 0 && p.M >= 512;
-  if (p.dw_big) {
+  // gemm_tn: enough workgroups to fill the chip, each split a multiple of 64 rows
+  const int tiles = (p.d / kGT) * (p.nt / (p.nt % 256 == 0 ? 256 : 128));
+  int s = 1;
+  while (s * tiles < 1024 && p.M % (2 * s * kGK) == 0) s *= 2;
+  p.dw = {s, p.M / s};
+  p.dw_big = {0, 0};
+  if (p.nt % kBigT == 0 && p.M >= 512) {
     // 256 x 256 tiles, one workgroup per CU: as many splits as fill the 256 CUs
     // once (a second, part-filled round costs more: eight splits of 42 tiles
     // 0.265 ms, six 0.206), of at least 128 rows; the last one may be shorter
-    const int tiles = (p.d / kBigT) * (p.nt / kBigT);
-    int s = tiles < 256 ? 256 / tiles : 1;
+    const int big = (p.d / kBigT) * (p.nt / kBigT);
+    s = big < 256 ? 256 / big : 1;
     if (s > p.M / 128) s = p.M / 128;
-    p.rows = (p.M / kBigK + s - 1) / s * kBigK;
-    p.splits = (p.M + p.rows - 1) / p.rows;
-  } else {
-    const int tiles = (p.d / kGT) * (p.nt / (p.nt % 256 == 0 ? 256 : 128));
-    int s = 1;
-    while (s * tiles < 1024 && p.M % (2 * s * kGK) == 0) s *= 2;
-    p.splits = s;
-    p.rows = p.M / s;
+    const int rows = (p.M / kBigK + s - 1) / s * kBigK;
+    p.dw_big = {(p.M + rows - 1) / rows, rows};
   }
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
   size_t off = 0;
@@ -955,7 +954,8 @@ static M2xPlan m2x_plan(const atomic_mamba2_proj_args* a, bool bwd) {
   if (bwd) {
     p.o_dpre = take(M * nt * 2);
     p.o_dxc = take(M * d * 2);
-    p.o_dw = take((size_t)p.splits * d * nt * 4);
+    // room for either GEMM: which one runs depends on x_bc's alignment
+    p.o_dw = take((size_t)(p.dw.n > p.dw_big.n ? p.dw.n : p.dw_big.n) * d * nt * 4);
     p.o_dbp = take((M / 32) * d * 4);
     p.o_dbs = take(d * 4);
     size_t so;
@@ -1064,14 +1064,17 @@ extern "C" int atomic_mamba2_proj_bwd(const atomic_mamba2_proj_args* a, const vo
     m2x_gemm_nt(g, e, aligned16({dx_bc}), st);
   });
   if (rc) return rc;
+  // the large tiles load their operands straight to LDS in 16-byte pieces
+  const bool dw_big = p.dw_big.n > 0 && aligned16({x_bc, dpre});
+  const M2xSplit dw = dw_big ? p.dw_big : p.dw;
   rc = L("m2p_dw_gemm", [&] {
-    const GemmTN g{(const bf16*)x_bc, (long long)a->in_stride, dpre, (long long)p.nt, p.d, p.nt, p.rows, dwp, p.M};
-    if (p.dw_big)
-      hipLaunchKernelGGL(gemm_tn_big, dim3((unsigned)(p.splits * (p.d / kBigT) * (p.nt / kBigT))), dim3(512), 0, st, g);
+    const GemmTN g{(const bf16*)x_bc, (long long)a->in_stride, dpre, (long long)p.nt, p.d, p.nt, dw.rows, dwp, p.M};
+    if (dw_big)
+      hipLaunchKernelGGL(gemm_tn_big, dim3((unsigned)(dw.n * (p.d / kBigT) * (p.nt / kBigT))), dim3(512), 0, st, g);
     else if (p.nt % 256 == 0)
-      hipLaunchKernelGGL(gemm_tn<256>, dim3((unsigned)(p.splits * (p.d / kGT) * (p.nt / 256))), dim3(256), 0, st, g);
+      hipLaunchKernelGGL(gemm_tn<256>, dim3((unsigned)(dw.n * (p.d / kGT) * (p.nt / 256))), dim3(256), 0, st, g);
     else
-      hipLaunchKernelGGL(gemm_tn<128>, dim3((unsigned)(p.splits * (p.d / kGT) * (p.nt / 128))), dim3(256), 0, st, g);
+      hipLaunchKernelGGL(gemm_tn<128>, dim3((unsigned)(dw.n * (p.d / kGT) * (p.nt / 128))), dim3(256), 0, st, g);
   });
   if (rc) return rc;
   rc = L("prologue_colsum", [&] {
@@ -1089,6 +1092,6 @@ extern "C" int atomic_mamba2_proj_bwd(const atomic_mamba2_proj_args* a, const vo
   if (rc) return rc;
   return L("m2p_dw_finish", [&] {
     hipLaunchKernelGGL(m2p_dw_finish, dim3((unsigned)(((size_t)p.d * p.nt + 255) / 256)), dim3(256), 0, st, p.d,
-                       p.n, p.splits, dwp, dbs, dw_dt, dw_b, dw_c, db_dt);
+                       p.n, dw.n, dwp, dbs, dw_dt, dw_b, dw_c, db_dt);
   });
 }

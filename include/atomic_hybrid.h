@@ -730,7 +730,9 @@ size_t atomic_mamba2_proj_workspace_size(const atomic_mamba2_proj_args* a, int b
 
 /*
  * Forward.
- *   x_bc : [B * L] rows of in_stride bf16 (d_inner used)
+ *   x_bc : [B * L] rows of in_stride bf16 (d_inner used).  Any base address
+ *   will do, here and in the backward; where x_bc, the workspace and the
+ *   outputs are 16-byte aligned the projections run in larger tiles.
  *   x, dt : [B, L, H, P] bf16   B, C : [B, L, N] bf16   A : [H] fp32
  *   dt_pre : [B, L, d_inner] bf16, b_pre / c_pre : [B, L, N] bf16 -- the
  *   projection outputs, written when non-NULL (the backward takes them)

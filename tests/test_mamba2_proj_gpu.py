@@ -133,3 +133,35 @@ def test_large_tiles_match_oracle_and_the_small_tiles(B, L, H, P, N):
     small, small_pres = PL.mamba2_proj_forward(gp[0, :256, :d].clone()[None], *gparams, H, save=True)
     for name, a, b in zip(OUTS[1:4] + PRES, outs[1:4] + pres, small[1:4] + small_pres):
         assert torch.equal(a[:1, :256], b), name
+
+
+@pytest.mark.parametrize("off,ws_off", [(4, 0), (0, 8)])
+def test_unaligned_operands_match_aligned_ones(off, ws_off):
+    """x_bc starting 4 columns into its tensor (8 bytes past a 16-byte address),
+    or a workspace 8 bytes past one, at sizes that otherwise take the large
+    tiles: the forward and dx bit for bit, the weight gradients (summed in
+    other row splits, then rounded to bf16) within one rounding of the largest."""
+    B, L, H, P, N = 3, 5632, 4, 128, 128
+    banner(f"mamba2 proj prologue unaligned x_bc+{off} workspace+{ws_off}")
+    d = H * P
+    wide, params, cots = _inputs(B, L, H, P, N, 17)
+    wide = torch.cat([wide, wide[..., :8]], -1).cuda()
+    gparams, gcots = [t.cuda() for t in params], [c.cuda() for c in cots]
+    view = wide[..., off:off + d]
+    assert view.data_ptr() % 16 == 2 * off
+    args = PL.mamba2_proj_make_args(B, L, H, P, N, wide.shape[-1])
+    ws = [torch.empty(_lib.load().atomic_mamba2_proj_workspace_size(args, i) + 8, dtype=torch.uint8,
+                      device="cuda")[ws_off:] for i in (0, 1)]
+    outs, pres = PL.mamba2_proj_forward(view, *gparams, H, save=True, workspace=ws[0])
+    grads = PL.mamba2_proj_backward(view, *gparams, H, pres, *gcots, workspace=ws[1])
+    dense = view.contiguous()
+    outs_d, pres_d = PL.mamba2_proj_forward(dense, *gparams, H, save=True)
+    grads_d = PL.mamba2_proj_backward(dense, *gparams, H, pres_d, *gcots)
+    torch.cuda.synchronize()
+    for name, a, b in zip(OUTS + PRES, outs + pres, outs_d + pres_d):
+        assert torch.equal(a, b), name
+    for name, a, b in zip(GRADS, grads, grads_d):
+        if name.startswith("dw_"):
+            assert rel_err(a, b) <= 2.0 ** -8, name
+        else:
+            assert torch.equal(a, b), name
