@@ -328,6 +328,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
     pf(2); pf(3);
     bare_barrier();
     for (int i = 0; i < dm.NT; ++i) { pf(i + 4); bare_barrier(); bare_barrier(); }
+    vm_wait<0>();  // nothing may still be on its way to this workgroup's LDS when it ends
     return;
   }
   if (wid >= 8 && wid < 8 + NL) {

@@ -683,6 +683,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
       bare_barrier();
       bare_barrier();
     }
+    vm_wait<0>();  // nothing may still be on its way to this workgroup's LDS when it ends
     return;
   }
   if (wid >= 8) {
