@@ -292,7 +292,8 @@ struct DhSeqLds {
 // B4 T8192 H16, fp32 dO: 0.340 -> 0.297 ms; B8 T4096 H6 0.159 -> 0.127 ms; B1
 // T32768 H16 0.761 -> 0.607 ms (0.769 without the prefetch wave); K = 64, B2
 // T4096 H16 0.081 -> 0.060 ms.
-template <typename TD, int C, int K, int V, int VT, int NL>
+// AL = false: a workspace that is not 16-byte aligned.
+template <typename TD, int C, int K, int V, int VT, int NL, bool AL = true>
 __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
     Gdn2Dims dm, Gdn2Chunks<bf16> ck, Gdn2Grads<bf16> gr, const TD* __restrict__ dO,
     const float* __restrict__ dh_final, float* __restrict__ dh0) {
@@ -337,11 +338,11 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
     auto issue = [&](int i) {
       const int n = last - i;
       unsigned char* b = lds + L::off_st + (i & 1) * L::ST;
-      dma_rows<K, NL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
-      dma_rows<K, NL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
-      dma_rows<K, NL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
-      dma_rows<C, NL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
-      if (lane < K / 4) dma16(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
+      dma_rows<K, NL, AL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
+      dma_rows<K, NL, AL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
+      dma_rows<K, NL, AL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
+      dma_rows<C, NL, AL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
+      if (lane < K / 4) copy16<AL>(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
     };
     // instructions of one chunk per wave: the wait that leaves only the newest chunk's outstanding
     constexpr int PER = (3 * C * L::RB + C * L::CB) / 1024 / NL + 1;
@@ -349,12 +350,12 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
     issue(0);
     if (last > 0) { issue(1); __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER)); }
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    bare_barrier();
+    loader_barrier<AL>();
     for (int i = 0; i < dm.NT; ++i) {
-      bare_barrier();
+      loader_barrier<AL>();
       if (i + 2 <= last) { issue(i + 2); __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER)); }
       else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-      bare_barrier();
+      loader_barrier<AL>();
     }
     return;
   }

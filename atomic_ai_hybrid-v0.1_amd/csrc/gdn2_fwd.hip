@@ -645,7 +645,8 @@ struct StateLds {
 // B1 T32768 H16: 0.825 -> 0.490 ms; B8 T4096 H6 with saves 0.175 -> 0.156 ms;
 // B4 T8192 H16 0.311 -> 0.248 ms, with saves 0.372 -> 0.348 ms; K = 64, B2
 // T4096 H16: 0.083 -> 0.038 ms.
-template <int C, int K, int V, int VT, int NL>
+// AL = false: per-chunk arrays that are not 16-byte aligned (a caller's own).
+template <int C, int K, int V, int VT, int NL, bool AL = true>
 __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
     Gdn2Dims dm, Gdn2Chunks<bf16> ck, const float* __restrict__ h0, float* __restrict__ o,
     float* __restrict__ h_final, int mode) {
@@ -691,20 +692,20 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
     const int lw = wid - 8;
     auto issue_ka = [&](int n) {
       unsigned char* b = lds + L::off_ka + (n % 3) * L::KA;
-      dma_rows<K, NL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
-      dma_rows<C, NL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
+      dma_rows<K, NL, AL>(ck.kg + (bh0 + n) * (C * K), b + L::s_kg, lw);
+      dma_rows<C, NL, AL>(ck.aqk + (bh0 + n) * (C * C), b + L::s_a, lw);
     };
     auto issue_wq = [&](int n) {
       unsigned char* b = lds + L::off_wq + (n & 1) * L::WQ;
-      dma_rows<K, NL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
-      dma_rows<K, NL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
+      dma_rows<K, NL, AL>(ck.wt + (bh0 + n) * (C * K), b + L::s_w, lw);
+      dma_rows<K, NL, AL>(ck.qg + (bh0 + n) * (C * K), b + L::s_q, lw);
       // u and gc_last: every wave issues the same number of instructions (it
       // counts them below), so a wave past the last piece repeats one
       constexpr int NI = C * L::UB / 1024, PU = VT / 8;
       static_assert(NI <= NL, "a wave loads one piece of u");
       const int ins = lw % NI, row = ins * (64 / PU) + lane / PU;
-      dma16(ck.u + (bh0 + n) * (C * V) + v0 + row * V + (lane % PU) * 8, b + L::s_u + ins * 1024);
-      if (lane < K / 4) dma16(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
+      copy16<AL>(ck.u + (bh0 + n) * (C * V) + v0 + row * V + (lane % PU) * 8, b + L::s_u + ins * 1024);
+      if (lane < K / 4) copy16<AL>(ck.gcl + (bh0 + n) * K + lane * 4, b + L::s_gl);
     };
     // instructions of one chunk per wave: the wait that leaves only the newest chunk's outstanding
     constexpr int PER = (3 * C * L::RB + C * L::CB) / 1024 / NL + 2;
@@ -718,18 +719,18 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
     } else {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     }
-    bare_barrier();
+    loader_barrier<AL>();
     for (int n = 0; n < dm.NT; ++n) {
       const bool more = n + 2 <= last;
       if (more) issue_ka(n + 2);   // its buffer was read last before step n - 1's first barrier
-      bare_barrier();
+      loader_barrier<AL>();
       if (more) {
         issue_wq(n + 2);           // its buffer was read last before this barrier
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER));
       } else {
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
       }
-      bare_barrier();
+      loader_barrier<AL>();
     }
     return;
   }

@@ -166,6 +166,12 @@ static Gdn2Chunks<T> gdn2_chunks(const Gdn2Plan& p, void* ws) {
   return c;
 }
 
+// Whether the arrays that the chunk loops load straight to LDS lie on 16-byte addresses.
+template <typename T>
+static bool gdn2_aligned(const Gdn2Chunks<T>& c) {
+  return aligned16({c.wt, c.qg, c.kg, c.aqk, c.u, c.gcl});
+}
+
 // Kernels A + B + C (gdn2_fwd_intra): the per-chunk intermediates into ck.
 template <typename T, int K, int ST = kIntraAll>
 static int gdn2_intra_launch(const Gdn2Plan& p, const void* q, const void* k, const void* v, const void* w,
@@ -193,6 +199,13 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
   const bool narrow = bh * (V / 16) <= 256;
   return L("gdn2_fwd_state", [&] {
     if constexpr (sizeof(T) == 2) {
+      // the loader waves' 16-byte loads to LDS need aligned arrays; a caller's own
+      // (or its workspace) may not be, and go through registers
+      if (!gdn2_aligned(ck)) {
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4, false>), dim3((unsigned)(bh * (V / 32))),
+                           dim3(512 + 64 * 4), 0, st, p.dm, ck, h0, o, h_final, mode);
+        return;
+      }
       // The prefetch wave while the workgroups leave CUs idle, where latency
       // bounds the step (B1 T32768 H16: 0.62 -> 0.49 ms, B8 T4096 H6 0.170 ->
       // 0.156); with 256 and more it only adds traffic (B4 T8192 H16: 0.248
@@ -268,7 +281,10 @@ static int gdn2_backward_impl(const Gdn2Plan& p, const void* q, const void* k, c
   rc = L("gdn2_bwd_dh", [&] {
     if constexpr (sizeof(T) == 2) {
       constexpr int NL = 2, NTHR = 512 + 64 * (NL + 3);
-      if (bh * (V / 16) <= 256)
+      if (!gdn2_aligned(ck))  // as in the forward state loop
+        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL, false>), dim3((unsigned)(bh * (V / VT))),
+                           dim3(512 + 64 * (NL + 2)), 0, st, p.dm, ck, gr, (const TD*)dO, dh_final, dh0);
+      else if (bh * (V / 16) <= 256)
         hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, 16, NL>), dim3((unsigned)(bh * (V / 16))), dim3(NTHR), 0, st,
                            p.dm, ck, gr, (const TD*)dO, dh_final, dh0);
       else

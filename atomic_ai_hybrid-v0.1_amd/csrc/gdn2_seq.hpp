@@ -65,17 +65,36 @@ __device__ __forceinline__ void store_frag_rows(bf16* dst, int ld, bf16x8 a) {
   *reinterpret_cast<u32x4*>(dst + (size_t)(l >> 2) * ld + 8 * (l & 3)) = q;
 }
 
+// dma16, or (AL = false) the same through registers, from any address.  The wave
+// that issues these has to see the LDS writes done too before the barrier.
+template <bool AL>
+__device__ __forceinline__ void copy16(const void* src, void* dst) {
+  if constexpr (AL) {
+    dma16(src, dst);
+  } else {
+    u32x4 v;
+    __builtin_memcpy(&v, src, 16);
+    *reinterpret_cast<u32x4*>(static_cast<unsigned char*>(dst) + lane_id() * 16) = v;
+  }
+}
+template <bool AL>
+__device__ __forceinline__ void loader_barrier() {
+  if constexpr (AL) bare_barrier();
+  else __syncthreads();
+}
+
 // Loader wave lw of NL: its share of a [64][K] bf16 block (row pieces permuted
 // as above); 64 K 2 / 1024 / NL instructions.
-template <int K, int NL>
+template <int K, int NL, bool AL>
 __device__ __forceinline__ void dma_rows(const bf16* src, unsigned char* dst, int lw) {
   constexpr int NP = K / 8, NI = 64 * K * 2 / 1024, RPI = 1024 / (2 * K);
   static_assert(NI % NL == 0, "the instructions split evenly over the loader waves");
-#pragma unroll
+  constexpr int UF = AL ? NI / NL : 4;  // through registers: few at a time
+#pragma unroll UF
   for (int i = 0; i < NI / NL; ++i) {
     const int ins = lw * (NI / NL) + i;
     const int row = ins * RPI + lane_id() / NP, slot = lane_id() % NP;
-    dma16(src + row * K + ((slot ^ (row & (NP - 1))) * 8), dst + ins * 1024);
+    copy16<AL>(src + row * K + ((slot ^ (row & (NP - 1))) * 8), dst + ins * 1024);
   }
 }
 // One of `parts` equal shares of an array's cache lines into L2.

@@ -3,6 +3,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+#include <initializer_list>
+
 #include "../../include/atomic_hybrid.h"
 
 namespace ah {
@@ -27,5 +30,12 @@ struct Launch {
     return ATOMIC_OK;
   }
 };
+
+// Whether every pointer lies on a 16-byte address (NULL does).
+inline bool aligned16(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (reinterpret_cast<uintptr_t>(p) & 15) return false;
+  return true;
+}
 
 }  // namespace ah

@@ -21,8 +21,6 @@
 // three following cotangents, recomputed past the tile's end).  Parameter
 // gradients: each workgroup (four consecutive tiles) combines its waves'
 // sums through LDS into one partial row; a final kernel sums the rows.
-#include <initializer_list>
-
 #include "../../include/atomic_hybrid.h"
 #include "common.hpp"
 #include "launch.hpp"
@@ -904,11 +902,6 @@ struct M2xPlan {
   M2xSplit dw, dw_big;  // gemm_tn's, gemm_tn_big's (n = 0: not for these sizes)
   size_t o_w, o_dpre, o_dxc, o_dw, o_dbp, o_dbs, o_conv, o_convsum, total;
 };
-static bool aligned16(std::initializer_list<const void*> ps) {
-  for (const void* p : ps)
-    if (reinterpret_cast<uintptr_t>(p) & 15) return false;
-  return true;
-}
 // C = A Bt^T over rows: 256 x 256 tiles where both sides divide and there are
 // more than 128 of them (with fewer, twice as many workgroups of 128 x 256
 // leave less of the chip idle), the outputs take 16-byte stores and the operands

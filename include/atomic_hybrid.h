@@ -282,7 +282,8 @@ int atomic_gdn2_recompute_wy(const atomic_gdn2_args* a, const void* q, const voi
 /* Kernel D: gdn2_inter_chunk_combine (kernel_d_pipeline.py:94-124), the
  * sequential state loop over those arrays.  h0 [B][H][K][V] (NULL: zeros) is
  * sanitised first like the reference's _sanitize_h0 (:54-55); o is written per
- * block, [B][H][NT][BT][V] fp32, and h_final [B][H][K][V] fp32. */
+ * block, [B][H][NT][BT][V] fp32, and h_final [B][H][K][V] fp32.  The bf16 arrays
+ * may start anywhere; all on 16-byte addresses run faster. */
 int atomic_gdn2_inter_chunk_combine(const atomic_gdn2_args* a, const void* Aqk, const void* w_pseudo,
                                     const void* u, const void* kg, const void* qg, const float* gc_last,
                                     const float* h0, float* o, float* h_final, void* stream);

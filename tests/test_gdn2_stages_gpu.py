@@ -247,3 +247,40 @@ def test_combine_with_state_and_residuals(dtype):
         assert res["h_pre_all"].shape == (NT, B, H, K, K) and e_h < tol and e_v < tol
         h = og.sanitize(h * torch.exp(gl_c)[..., None] + kg_c.transpose(-1, -2) @ v_new)
     assert set(res) == {"Aqk", "Akk", "A", "h_pre_all", "v_new_all", "w_pseudo", "u", "kg", "qg", "gc_last"}
+
+
+def _off8(t):
+    """t's values in memory that starts 8 bytes past a 16-byte address."""
+    n = 8 // t.element_size()
+    out = torch.empty(t.numel() + n, dtype=t.dtype, device=t.device)[n:].view(t.shape)
+    assert out.data_ptr() % 16 == 8
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("K", [64, 128])
+def test_unaligned_chunk_arrays_match_aligned_ones(K):
+    """Kernel D on caller-owned bf16 arrays that are not 16-byte aligned (all of
+    them, and gc_last alone), bit for bit the aligned call's results; and the
+    whole forward and backward with such a workspace."""
+    B, T, H = 2, 320, 3
+    banner(f"gdn2 unaligned chunk arrays K{K}")
+    q, k, v, w, b, g = (t.cuda() for t in _inputs(B, T, H, K, BF16, 57))
+    h0 = 0.4 * torch.randn(B, H, K, K, generator=torch.Generator().manual_seed(58)).cuda()
+    Aqk, _, wp, u, kg, qg, gl = KD.build_chunk_wy(q, k, v, w, b, g, 0.6)
+    arrays = (Aqk, wp, u, kg, qg, gl)
+    ref = KD.gdn2_inter_chunk_combine_with_state(*arrays, 0.6, h0=h0)
+    for got in (tuple(_off8(t) for t in arrays), arrays[:5] + (_off8(gl),)):
+        out = KD.gdn2_inter_chunk_combine_with_state(*got, 0.6, h0=h0)
+        torch.cuda.synchronize()
+        for x, y in zip(out, ref):
+            assert torch.equal(x, y)
+    do = torch.randn(B, T, H, K, generator=torch.Generator().manual_seed(59)).cuda()
+    runs = []
+    for off in (0, 8):
+        n = G.workspace_bytes(G.make_args(q, v, 0.6))
+        ws = torch.empty(n + 8, dtype=torch.uint8, device="cuda")[off:]
+        o, h, ws = G.forward(q, k, v, w, b, g, 0.6, h0=h0, save=True, workspace=ws)
+        runs.append((o, h) + tuple(G.backward(q, k, v, w, b, g, 0.6, do, h0=h0, workspace=ws, reuse=True)))
+    torch.cuda.synchronize()
+    for x, y in zip(*runs):
+        assert (x is None and y is None) or torch.equal(x, y)
