@@ -632,22 +632,28 @@ struct StateLds {
 };
 
 // bf16 state loop of one (batch, head, VT columns): waves 0-3 compute v_new
-// and the state, 4-7 o (and store the saves), the next NL load the chunks (see
-// gdn2_seq.hpp), and one more, when launched, touches the lines of the chunk
-// kPrefetch steps on: it hides the memory latency that two chunks in flight do
-// not cover.
+// and the state, 4-7 o, the next NL load the chunks (see gdn2_seq.hpp), two more
+// store the saves (32 columns), and a last one, when launched, touches the lines
+// of the chunk kPrefetch steps on: it hides the memory latency that two chunks in
+// flight do not cover.
 // v_new and the state are computed transposed (columns of h as MFMA rows), so
 // a lane's four results are four consecutive columns of one row of the LDS
 // copies.  Bound by the step's chain of LDS reads, MFMAs and two barriers when
 // the operands come from L2 (0.87 us a chunk at 16 columns, 1.3 at 32, K =
 // 128; the former kernel, in which every wave loaded, staged and computed,
 // 1.40 and 1.7), and by HBM with 256 workgroups and the saves.
-// B1 T32768 H16: 0.825 -> 0.490 ms; B8 T4096 H6 with saves 0.175 -> 0.156 ms;
-// B4 T8192 H16 0.311 -> 0.248 ms, with saves 0.372 -> 0.348 ms; K = 64, B2
-// T4096 H16: 0.083 -> 0.038 ms.
+// Kernel times, former -> now: B1 T32768 H16 0.822 -> 0.514 ms, with saves 0.902
+// -> 0.617; B8 T4096 H6 with saves 0.172 -> 0.155; B4 T8192 H16 0.270 -> 0.231,
+// with saves 0.329 -> 0.318; K = 64 with saves, B2 T4096 H16 0.097 -> 0.071, B8
+// T4096 H16 0.135 -> 0.135.
+// The saves at 32 columns: as 64-byte row pieces by the o waves, inside their MFMA
+// chain, they took the same bytes 0.344 ms at B4 T8192 H16 (the pieces by waves of
+// their own 0.348), as whole rows 0.318.  At 16 columns latency bounds the step
+// and more waves reading LDS lengthen it (B1 T32768 H16: 0.634 against 0.617), so
+// there the o waves store them.
 // AL = false: per-chunk arrays that are not 16-byte aligned (a caller's own).
 template <int C, int K, int V, int VT, int NL, bool AL = true>
-__global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
+__global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_fwd_state(
     Gdn2Dims dm, Gdn2Chunks<bf16> ck, const float* __restrict__ h0, float* __restrict__ o,
     float* __restrict__ h_final, int mode) {
   typedef StateLds<C, K, VT> L;
@@ -666,7 +672,9 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
   unsigned char* sH = lds + L::off_h;
   unsigned char* sVn = lds + L::off_vn;
 
-  if (wid == 8 + NL) {
+  const bool save = (mode & kStateSave) != 0;
+  const int nsave = VT == 32 && save ? 2 : 0;
+  if (wid == 8 + NL + nsave) {
     // ---------------- L2 prefetch: the V tiles of a head share an XCD and split its lines
     auto prefetch = [&](int n) {
       if (n > last) return;
@@ -685,6 +693,26 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
       bare_barrier();
     }
     vm_wait<0>();  // nothing may still be on its way to this workgroup's LDS when it ends
+    return;
+  }
+  if (VT == 32 && wid >= 8 + NL) {
+    // ---------------- the saves, state and v_new transposed: a column block a wave
+    const int sw = wid - 8 - NL;
+    auto put = [&](const unsigned char* src, bf16* dst, auto nk) {
+      constexpr int NK = decltype(nk)::value;  // k blocks of 32 columns
+      bf16x8 a[NK];
+#pragma unroll
+      for (int s = 0; s < NK; ++s) a[s] = seq_colfrag<VT>(src, sw, 32 * s);
+#pragma unroll
+      for (int i = 0; i < NK; ++i) store_frags_1k<NK>(dst + (size_t)(v0 + 16 * sw) * (32 * NK), i, a);
+    };
+    __syncthreads();
+    for (int n = 0; n < dm.NT; ++n) {
+      put(sH, ck.hT + (bh0 + n) * (V * K), std::integral_constant<int, XK>());
+      __syncthreads();
+      put(sVn, ck.vnT + (bh0 + n) * (V * C), std::integral_constant<int, XC>());
+      __syncthreads();
+    }
     return;
   }
   if (wid >= 8) {
@@ -815,8 +843,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
             h_final[((size_t)bh * K + 16 * (w * RB + t) + r16) * V + v0 + 16 * u + 4 * g4 + i] = hs[t][u][i];
     }
   } else {
-    // ---------------- o = scale qg h + Aqk v_new (rows 16 w ...), and the saves
-    const bool save = (mode & kStateSave) != 0;
+    // ---------------- o = scale qg h + Aqk v_new (rows 16 w ...)
     const bool chunk_o = (mode & kStateChunkO) != 0;
     const size_t ors = chunk_o ? (size_t)V : (size_t)dm.H * V;  // o's row stride
     __syncthreads();
@@ -834,7 +861,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
         for (int u = 0; u < NTI; ++u) {
           const bf16x8 a = seq_colfrag<VT>(sH, u, 32 * s);
           x[u] = M::mma(qf, a, x[u]);
-          if (save && s == w) store_frag_rows(ck.hT + bhn * V * K + (size_t)(v0 + 16 * u) * K + 32 * s, K, a);
+          if (VT == 16 && save && s == w) store_frag_rows(ck.hT + bhn * V * K + (size_t)v0 * K + 32 * s, K, a);
         }
       }
 #pragma unroll
@@ -851,7 +878,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 1)) void gdn2_fwd_state(
         for (int u = 0; u < NTI; ++u) {
           const bf16x8 a = seq_colfrag<VT>(sVn, u, 32 * s);
           if (32 * s <= 16 * w + 15) x[u] = M::mma(af[s], a, x[u]);  // Aqk is lower triangular
-          if (save && s == w) store_frag_rows(ck.vnT + bhn * V * C + (size_t)(v0 + 16 * u) * C + 32 * s, C, a);
+          if (VT == 16 && save && s == w) store_frag_rows(ck.vnT + bhn * V * C + (size_t)v0 * C + 32 * s, C, a);
         }
       if (o) {
         float* og = chunk_o ? o + bhn * C * V + v0 : o + (((size_t)bb * dm.T + (size_t)n * C) * dm.H + h) * V + v0;

@@ -199,11 +199,12 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
   const bool narrow = bh * (V / 16) <= 256;
   return L("gdn2_fwd_state", [&] {
     if constexpr (sizeof(T) == 2) {
+      const int ns = mode & kStateSave ? 2 : 0;  // waves that store the saves (32 columns)
       // the loader waves' 16-byte loads to LDS need aligned arrays; a caller's own
       // (or its workspace) may not be, and go through registers
       if (!gdn2_aligned(ck)) {
         hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4, false>), dim3((unsigned)(bh * (V / 32))),
-                           dim3(512 + 64 * 4), 0, st, p.dm, ck, h0, o, h_final, mode);
+                           dim3(512 + 64 * (4 + ns)), 0, st, p.dm, ck, h0, o, h_final, mode);
         return;
       }
       // The prefetch wave while the workgroups leave CUs idle, where latency
@@ -216,7 +217,7 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
                            p.dm, ck, h0, o, h_final, mode);
       } else {
         const unsigned nwg = (unsigned)(bh * (V / 32));
-        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg), dim3(512 + 64 * (4 + (nwg < 256))), 0, st,
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg), dim3(512 + 64 * (4 + ns + (nwg < 256))), 0, st,
                            p.dm, ck, h0, o, h_final, mode);
       }
     } else {

@@ -65,6 +65,25 @@ __device__ __forceinline__ void store_frag_rows(bf16* dst, int ld, bf16x8 a) {
   *reinterpret_cast<u32x4*>(dst + (size_t)(l >> 2) * ld + 8 * (l & 3)) = q;
 }
 
+// Kilobyte i of the 16 rows of 32 NK columns that NK fragments hold, rows dense:
+// lane l's 16 bytes of it come from fragment (piece / 4), lane (row, piece & 3).
+template <int NK>
+__device__ __forceinline__ void store_frags_1k(bf16* dst, int i, const bf16x8 (&a)[NK]) {
+  constexpr int PP = 4 * NK;  // pieces a row
+  const int e = 64 * i + lane_id(), pc = e % PP, from = 4 * (e / PP + 16 * (pc & 3));
+  u32x4 q = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int s = 0; s < NK; ++s) {
+    const u32x4 p = __builtin_bit_cast(u32x4, a[s]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t x = __builtin_amdgcn_ds_bpermute(from, p[j]);
+      q[j] = (pc >> 2) == s ? x : q[j];
+    }
+  }
+  *reinterpret_cast<u32x4*>(dst + e * 8) = q;
+}
+
 // dma16, or (AL = false) the same through registers, from any address.  The wave
 // that issues these has to see the LDS writes done too before the barrier.
 template <bool AL>
