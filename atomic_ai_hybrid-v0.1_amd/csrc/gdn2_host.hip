@@ -185,7 +185,17 @@ static int gdn2_intra_launch(const Gdn2Plan& p, const void* q, const void* k, co
   });
 }
 
-// Kernel D (gdn2_fwd_state) over the intermediates in ck; mode: kState* bits.
+// Whether the chunk loops' V tiles of one head land on one XCD (xcd_group_map).
+static bool gdn2_tiles_share_l2(int bh) { return bh % 8 == 0; }
+// 16-column tiles in the bf16 chunk loops: up to a workgroup per CU, or three to
+// every four CUs where the tiles of a head do not share an L2 and each fetches the
+// chunk's operands for itself (T2048 K = 128 forward / with saves / dh: 20 heads
+// 49 / 53 / 55 us against 45 / 64 / 56 with 32 columns, 25 heads 62 / 68 / 65
+// against 46 / 65 / 57, 31 heads 79 / 90 / 84 against 45 / 76 / 59; K = 64, 41
+// heads 33 / 36 / 40 against 30 / 39 / 40, 50 heads 41 / 46 / 43 against 31 / 44 / 41).
+static bool gdn2_narrow(int bh, int V) { return bh * (V / 16) <= (gdn2_tiles_share_l2(bh) ? 256 : 192); }
+
+// Kernels A + B + C (gdn2_fwd_intra): the) over the intermediates in ck; mode: kState* bits.
 template <typename T, int K>
 static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const float* h0, float* o,
                              float* h_final, int mode, Launch& L) {
@@ -196,7 +206,7 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
   // chunk step is shorter and twice the workgroups walk the chunks; every tile
   // re-reads the chunk's w, q, kg, which its XCD's L2 serves.  Past that, 32
   // (B4 T8192 H16 K = 128 without saves: 0.36 ms with 16, 0.25 with 32).
-  const bool narrow = bh * (V / 16) <= 256;
+  const bool narrow = sizeof(T) == 2 ? gdn2_narrow(bh, V) : bh * (V / 16) <= 256;
   return L("gdn2_fwd_state", [&] {
     if constexpr (sizeof(T) == 2) {
       const int ns = mode & kStateSave ? 2 : 0;  // waves that store the saves (32 columns)
@@ -207,18 +217,22 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
                            dim3(512 + 64 * (4 + ns)), 0, st, p.dm, ck, h0, o, h_final, mode);
         return;
       }
-      // The prefetch wave while the workgroups leave CUs idle, where latency
-      // bounds the step (B1 T32768 H16: 0.62 -> 0.49 ms, B8 T4096 H6 0.170 ->
-      // 0.156); with 256 and more it only adds traffic (B4 T8192 H16: 0.248
-      // without, 0.258 with).
+      // The prefetch wave where the tiles of a head share an L2 (elsewhere each
+      // XCD gets only its share of the lines: B3 T4096 H21, 32 columns, 0.212 ms
+      // with it, 0.173 without), and with 32 columns only while the workgroups
+      // leave CUs idle, where latency bounds the step (B8 T4096 H6 with saves
+      // 0.155 ms with it, 0.168 without; B4 T4096 H16, 256 workgroups, 0.136 and
+      // 0.130).  With 16 columns it pays up to all 256 CUs (B1 T8192 H32: 0.159
+      // and 0.210 ms, with saves 0.193 and 0.278; B1 T32768 H16: 0.51 and 0.62).
+      const bool shared = gdn2_tiles_share_l2(bh);
       if (narrow) {
         const unsigned nwg = (unsigned)(bh * (V / 16));
-        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 16, 2>), dim3(nwg), dim3(512 + 64 * (2 + (nwg < 256))), 0, st,
-                           p.dm, ck, h0, o, h_final, mode);
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 16, 2>), dim3(nwg), dim3(512 + 64 * (2 + shared)), 0, st, p.dm, ck,
+                           h0, o, h_final, mode);
       } else {
         const unsigned nwg = (unsigned)(bh * (V / 32));
-        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg), dim3(512 + 64 * (4 + ns + (nwg < 256))), 0, st,
-                           p.dm, ck, h0, o, h_final, mode);
+        hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg),
+                           dim3(512 + 64 * (4 + ns + (shared && nwg < 256))), 0, st, p.dm, ck, h0, o, h_final, mode);
       }
     } else {
       if (narrow)
@@ -278,19 +292,25 @@ static int gdn2_backward_impl(const Gdn2Plan& p, const void* q, const void* k, c
   const int bh = p.dm.B * p.dm.H;
   const unsigned nblk = (unsigned)p.bhn;
   // 16-column V tiles under the same condition as the forward state loop (B4
-  // T8192 H16 K = 128: 0.39 ms with 16, 0.30 with 32)
+  // T8192 H16 K = 128: 0.39 ms with 16, 0.30 with 32).  The prefetch wave too,
+  // except that at K = 128 it pays with 32 columns and a full chip as well (B4
+  // T8192 H16 0.264 ms with it, 0.278 without; B8 T4096 H24 0.402 and 0.424; at K =
+  // 64, B8 T4096 H16, 0.128 and 0.116).
   rc = L("gdn2_bwd_dh", [&] {
     if constexpr (sizeof(T) == 2) {
-      constexpr int NL = 2, NTHR = 512 + 64 * (NL + 3);
-      if (!gdn2_aligned(ck))  // as in the forward state loop
-        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL, false>), dim3((unsigned)(bh * (V / VT))),
-                           dim3(512 + 64 * (NL + 2)), 0, st, p.dm, ck, gr, (const TD*)dO, dh_final, dh0);
-      else if (bh * (V / 16) <= 256)
-        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, 16, NL>), dim3((unsigned)(bh * (V / 16))), dim3(NTHR), 0, st,
-                           p.dm, ck, gr, (const TD*)dO, dh_final, dh0);
+      constexpr int NL = 2, NT0 = 512 + 64 * (NL + 2);
+      const bool al = gdn2_aligned(ck), narrow = al && gdn2_narrow(bh, V);
+      const unsigned nwg = (unsigned)(bh * (V / (narrow ? 16 : VT)));
+      const unsigned nthr = NT0 + 64 * (gdn2_tiles_share_l2(bh) && (narrow || K == 128 || nwg < 256));
+      if (!al)  // as in the forward state loop
+        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL, false>), dim3(nwg), dim3(NT0), 0, st, p.dm, ck, gr,
+                           (const TD*)dO, dh_final, dh0);
+      else if (narrow)
+        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, 16, NL>), dim3(nwg), dim3(nthr), 0, st, p.dm, ck, gr,
+                           (const TD*)dO, dh_final, dh0);
       else
-        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL>), dim3((unsigned)(bh * (V / VT))), dim3(NTHR), 0, st,
-                           p.dm, ck, gr, (const TD*)dO, dh_final, dh0);
+        hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL>), dim3(nwg), dim3(nthr), 0, st, p.dm, ck, gr,
+                           (const TD*)dO, dh_final, dh0);
     } else {
       hipLaunchKernelGGL((gdn2_bwd_dh_f32<T, TD, C, K, V, VT>), dim3((unsigned)(bh * (V / VT))), dim3(512), 0, st,
                          p.dm, ck, gr, (const TD*)dO, dh_final, dh0);

@@ -71,24 +71,30 @@ def test_backward_matches_autodiff(B, T, H, K, dtype, scale, with_state, reuse):
 
 
 @pytest.mark.parametrize("T", [64, 448])
-@pytest.mark.parametrize("dtype,K,B,H", [(F32, 64, 5, 13), (F32, 128, 3, 11), (BF16, 64, 5, 13), (BF16, 128, 3, 11)])
+@pytest.mark.parametrize("dtype,K,B,H", [
+    (F32, 64, 5, 13), (F32, 128, 3, 11), (BF16, 64, 5, 13), (BF16, 128, 3, 11),
+    (BF16, 64, 7, 7), (BF16, 128, 5, 5),     # 49, 25: not a multiple of 8, so above 192 already
+    (BF16, 64, 8, 8), (BF16, 128, 4, 8),     # 256 workgroups of 16 columns, with the prefetch wave
+    (BF16, 64, 16, 8), (BF16, 128, 8, 8),    # 256 of 32 columns, with it (dh at K = 128) and without
+])
 def test_wide_state_loops_past_the_narrow_ones(dtype, K, B, H, T):
     """The smallest B H whose chunk loops take 32 columns a workgroup (B H K / 16
-    above 256) in every dtype and head size, one chunk and seven: forward and
-    backward against the oracle, and bit for bit against the same batches in
-    two calls, which take 16 columns."""
+    above 256, in bf16 above 192 where B H is not a multiple of 8) in every
+    dtype and head size, and the fullest launches on both sides, one chunk and
+    seven: forward and backward against the oracle, and bit for bit against
+    the same batches in two calls, which take 16 columns."""
     banner(f"gdn2 wide loops {dtype} K{K} B{B} H{H} T{T}")
     args, ref = _case(B, T, H, K, dtype, seed=29 + K, scale=0.7, with_state=True)
     q, k, v, w, b, g, dO, h0, dh = args
     o_ref, h_ref = og.gdn2_chunked_wy_reference(q, k, v, g, b, w, 0.7, 64, h0=h0)
     dev = [t.cuda() for t in args]
     outs = []
-    for sl in (slice(0, B), slice(0, B - 1 - B // 4), slice(B - 1 - B // 4, B)):
+    cut = B // 2 + B % 2
+    for sl in (slice(0, B), slice(0, cut), slice(cut, B)):
         *x, do, h, d = (t[sl] for t in dev)
         o, hf, ws = G.forward(*x, 0.7, h0=h, save=True)
         outs.append((o, hf) + tuple(G.backward(*x, 0.7, do, dh_final=d, h0=h, workspace=ws, reuse=True)))
     torch.cuda.synchronize()
-    assert B * H * K // 16 > 256 and all(t[0].shape[0] * H * K // 16 <= 256 for t in outs[1:])
     for name, whole, lo, hi in zip(("o", "h_final") + tuple(NAMES), *outs):
         assert torch.equal(whole, torch.cat([lo, hi])), name
     tol = tol_for(dtype)
