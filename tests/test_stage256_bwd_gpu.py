@@ -312,3 +312,27 @@ def test_mamba2_bwd_scan_and_da_match_the_oracle(C, P, N, dy_dtype):
     torch.cuda.synchronize()
     for n, g_, r in zip(("ddt", "dB", "dC", "dx", "dA", "dstate0"), comp, mb0):
         _check(f"composed vs MB0 {n}", g_, om.final_sanitize(r))
+
+
+def test_mb2_masked_pairs_of_a_huge_dy_count():
+    """A finite dy whose product with a masked partner's dBx overflows: the
+    zero weight makes it NaN, which the clip after the sum turns into 0, on the
+    row side (row 3) and the column side (row 40), also where the partner lies
+    in another wave's rows."""
+    banner("mamba2 MB2 masked pairs of a huge dy")
+    B, T, H, P, N, C, p = 1, 64, 1, 64, 64, 64, 5
+    gen = torch.Generator().manual_seed(12)
+    Bm, Cm = (torch.randn(B, T, N, generator=gen) for _ in range(2))
+    dt = torch.ones(B, T, H, P)
+    x, dy = torch.zeros(B, T, H, P), torch.zeros(B, T, H, P)
+    x[0, 1, 0, p], x[0, 40, 0, p] = 1e-34, 1e4
+    dy[0, 3, 0, p], dy[0, 50, 0, p] = 1e36, 1.0
+    cum = -0.01 * torch.arange(1, C + 1).float()[None, None, None, :, None].expand(B, H, 1, C, P).contiguous()
+    zero = torch.zeros(B, H, 1, P, N)
+    run = lambda d: MB2.intra_chunk_ssd_bwd_pallas(dt.cuda(), x.cuda(), Bm.cuda(), Cm.cuda(), cum.cuda(), d.cuda(),
+                                                   zero.cuda(), C)[-1].cpu().reshape(C, P)
+    dcum = run(dy)
+    assert dcum[3, p] == 0 and dcum[40, p] == 0
+    dy[0, 3, 0, p] = 1e33   # no overflow: the same pairs' other terms are there
+    dcum = run(dy)
+    assert dcum[3, p] != 0 and dcum[40, p] != 0
