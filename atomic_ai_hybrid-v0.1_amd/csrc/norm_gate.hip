@@ -375,9 +375,9 @@ static int ng_check(const atomic_norm_gate_args* a) {
   return ATOMIC_OK;
 }
 
-// gate's row stride: at least a row, whole 16-byte pieces
+// gate's row stride: at least a row, whole 16-byte pieces, byte offsets of all rows in 63 bits
 static int ng_stride_check(const atomic_norm_gate_args* a, int64_t gate_stride, const void* gate) {
-  if (gate_stride < a->dim || gate_stride % 8 != 0 || gate_stride > (1LL << 30)) return ATOMIC_ERR_SHAPE;
+  if (gate_stride < a->dim || gate_stride % 8 != 0 || gate_stride > INT64_MAX / 2 / a->rows) return ATOMIC_ERR_SHAPE;
   if (gate_stride != a->dim && ((uintptr_t)gate & 15) != 0) return ATOMIC_ERR_SHAPE;
   return ATOMIC_OK;
 }

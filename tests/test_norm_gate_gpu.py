@@ -99,6 +99,23 @@ def test_gate_read_in_place_matches_a_dense_gate(variant, ovar, B, T, d, width, 
         assert a.shape == b.shape and torch.equal(a, b)
 
 
+def test_gate_rows_far_apart():
+    """Rows of the gate more than 2^30 elements apart (one batch row of a
+    transposed tensor) give the dense gate's results."""
+    banner("norm_gate distant gate rows")
+    d, ld = 512, (1 << 30) + 8
+    wide = torch.zeros(ld + d, dtype=torch.bfloat16, device="cuda")
+    gate = wide.as_strided((1, 2, d), (8, ld, 1))
+    gen = torch.Generator().manual_seed(31)
+    gate.copy_(torch.randn(1, 2, d, generator=gen))
+    x, w = torch.randn(1, 2, d, generator=gen).cuda(), (1.0 + 0.1 * torch.randn(d, generator=gen)).cuda()
+    dout = torch.randn(1, 2, d, generator=gen).to(torch.bfloat16).cuda()
+    got = (NG.forward(x, gate, w, NG.MAMBA2), *NG.backward(x, gate, w, dout, NG.MAMBA2))
+    gate = gate.contiguous()
+    for a, b in zip(got, (NG.forward(x, gate, w, NG.MAMBA2), *NG.backward(x, gate, w, dout, NG.MAMBA2))):
+        assert torch.equal(a, b)
+
+
 def test_unsupported_dimension_is_rejected_before_launch():
     banner("norm_gate shape error")
     x = torch.zeros(4, 640, device="cuda")
