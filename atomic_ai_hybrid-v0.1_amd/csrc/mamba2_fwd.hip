@@ -374,6 +374,9 @@ __global__ __launch_bounds__(256) void mamba2_state_pass(Mamba2Dims dm, Mamba2Ch
     st.z = sanitize(st.z * dce + src[k].z);
     st.w = sanitize(st.w * dce + src[k].w);
     load(k, min(it + D, NT - 1));
+    // a step's loads stay behind its predecessor's, or a wait takes the next steps' too
+    // (B2 T16128 H2 P128 N128: 0.023 -> 0.018 ms; the backward 0.046 -> 0.047)
+    if constexpr (!BWD) __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
   for (int k = 0; k < D; ++k) load(k, min(k, NT - 1));
