@@ -95,10 +95,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int NTH = (K / 16) * NTI;  // dh tiles
   constexpr int TPW = NTH / NW;
   constexpr int NTV = (C / 16) * NTI;  // dv_new tiles
-  // with fewer dv_new tiles than waves (16-column V tiles) the first NTV waves take one each
-  constexpr int VPW = NTV >= NW ? NTV / NW : 1;
-  static_assert(NTH % NW == 0 && (NTV % NW == 0 || NW % NTV == 0) && TPW >= 1,
-                "tiles must split evenly over the waves");
+  constexpr int VPW = NTV / NW;
+  static_assert(NTH % NW == 0 && NTV % NW == 0 && TPW >= 1 && VPW >= 1, "tiles must split evenly over the waves");
   // tiles of one row block computed together (sharing their A fragments)
   constexpr int GV = VPW < NTI ? VPW : NTI, GT = TPW < NTI ? TPW : NTI;
   static_assert(VPW % GV == 0 && NTI % GV == 0 && TPW % GT == 0 && NTI % GT == 0, "tile groups");
@@ -189,7 +187,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
       // dv_new = sanitize(Aqk^T dO + kg dh)   (b2:70, b1:30-32)
   #pragma unroll
-      for (int gi = 0; gi < ((NTV >= NW || wv_id < NTV) ? VPW / GV : 0); ++gi) {
+      for (int gi = 0; gi < VPW / GV; ++gi) {
         const int tile0 = wv_id * VPW + gi * GV, mj = tile0 / NTI, ni0 = tile0 % NTI;
         const int k0 = tri_k0<T>(mj);
         f32x4 acc[GV];
@@ -475,7 +473,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
         store4(reinterpret_cast<bf16*>(sDh + seq_off<VT>(16 * w + r16, 16 * u + 4 * g4)), hs[u]);
       }
     }
-    // dv_new rows out (LDS holds them negated): 16-byte pieces over the eight waves
+    // dv_new rows out (LDS holds them negated): a 16-byte piece for each of the first C VT / 8 threads
     {
       constexpr int PPR = VT / 8;
       const int e = threadIdx.x;

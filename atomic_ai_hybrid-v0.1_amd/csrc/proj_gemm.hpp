@@ -351,7 +351,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kBigS * 2 * SB];
   const int w = wave_id(), lane = lane_id();
   const int ntn = g.N / kBigT, ntk = g.Kd / kBigT;
-  // the tiles of one split share its rows: splits over the XCDs
+  // one split's tiles are consecutive workgroups: they read the same rows at the same
+  // time (each XCD fetches them once, since consecutive workgroups go over all XCDs)
   const int tiles = ntk * ntn;
   const int s = blockIdx.x / tiles, tt = blockIdx.x % tiles;
   const int tk = tt / ntn, tn = tt % ntn;

@@ -205,12 +205,12 @@ __device__ __forceinline__ void conv_fwd_tile(const PlDims& dm, const bf16* __re
   }
 }
 
-template <int MODE, int DH>
+// One convolution without a norm or clip (the Mamba2 block's x).
 __global__ __launch_bounds__(256) void prologue_conv_fwd(PlDims dm, const bf16* __restrict__ lin,
                                                          const float* __restrict__ conv_w,
                                                          const float* __restrict__ conv_b,
                                                          bf16* __restrict__ out) {
-  conv_fwd_tile<MODE, DH>(dm, lin, conv_w, conv_b, out);
+  conv_fwd_tile<kPlain, 128>(dm, lin, conv_w, conv_b, out);
 }
 
 // The GDN2 block's three convolutions in one launch (blockIdx.y = q, k, v).
@@ -421,11 +421,10 @@ __device__ __forceinline__ void conv_bwd_tile(const PlDims& dm, const bf16* __re
   combine_partials<NV, CPL>(acc, part + ((size_t)b * ngrp + grp) * dm.d * NV, c);
 }
 
-template <int MODE, int DH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void prologue_conv_bwd(
     PlDims dm, const bf16* __restrict__ lin, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
     const bf16* __restrict__ dout, bf16* __restrict__ dlin, float* __restrict__ part) {
-  conv_bwd_tile<MODE, DH>(dm, lin, conv_w, conv_b, dout, dlin, part);
+  conv_bwd_tile<kPlain, 128>(dm, lin, conv_w, conv_b, dout, dlin, part);
 }
 
 // The three convolutions of the GDN2 block in one launch, as in the forward.
@@ -819,7 +818,7 @@ extern "C" int atomic_mamba2_prologue_fwd(const atomic_mamba2_prologue_args* a, 
   Launch L{a->profile, st};
   const unsigned nconv = (unsigned)(((size_t)dm.B * (dm.L / kTileF) * (dm.d / 512) + 3) / 4);
   rc = L("prologue_conv_fwd", [&] {
-    hipLaunchKernelGGL((prologue_conv_fwd<kPlain, 128>), dim3(nconv), dim3(256), 0, st, dm, (const bf16*)x_bc,
+    hipLaunchKernelGGL(prologue_conv_fwd, dim3(nconv), dim3(256), 0, st, dm, (const bf16*)x_bc,
                        conv_w, conv_b, (bf16*)x);
   });
   if (rc) return rc;
@@ -854,7 +853,7 @@ extern "C" int atomic_mamba2_prologue_bwd(const atomic_mamba2_prologue_args* a, 
   Launch L{a->profile, st};
   const int ngrp = dm.L / (4 * kTileB);
   rc = L("prologue_conv_bwd", [&] {
-    hipLaunchKernelGGL((prologue_conv_bwd<kPlain, 128>), dim3((unsigned)((size_t)dm.B * ngrp * (dm.d / (64 * kCplB)))),
+    hipLaunchKernelGGL(prologue_conv_bwd, dim3((unsigned)((size_t)dm.B * ngrp * (dm.d / (64 * kCplB)))),
                        dim3(256), 0, st, dm, (const bf16*)x_bc, conv_w, conv_b, (const bf16*)dx, (bf16*)dx_bc, part);
   });
   if (rc) return rc;
@@ -903,8 +902,10 @@ struct M2xPlan {
   size_t o_w, o_dpre, o_dxc, o_dw, o_dbp, o_dbs, o_conv, o_convsum, total;
 };
 // C = A Bt^T over rows: 256 x 256 tiles where both sides divide and there are
-// more than 128 of them (with fewer, twice as many workgroups of 128 x 256
-// leave less of the chip idle), the outputs take 16-byte stores and the operands
+// more than 128 of them (up to 128, twice as many workgroups of 128 x 256 fit
+// the chip at once too and take as long: 1792 columns of K 1536, 126 tiles 61.1 and
+// 62.2 us, 140 tiles 61.7 and 80.0; 768 of 512, 96 tiles 36.3 and 36.3, 132 tiles
+// 37.0 and 43.7), the outputs take 16-byte stores and the operands
 // 16-byte loads to LDS (gemm_nt loads to registers, from any address).
 template <typename Epi>
 static void m2x_gemm_nt(const GemmNT& g, const Epi& e, bool aligned, hipStream_t st) {
@@ -987,7 +988,7 @@ extern "C" int atomic_mamba2_proj_fwd(const atomic_mamba2_proj_args* a, const vo
   if (rc) return rc;
   rc = L("prologue_conv_fwd", [&] {
     const unsigned nconv = (unsigned)(((size_t)p.dm.B * (p.dm.L / kTileF) * (p.d / 512) + 3) / 4);
-    hipLaunchKernelGGL((prologue_conv_fwd<kPlain, 128>), dim3(nconv), dim3(256), 0, st, p.dm, (const bf16*)x_bc,
+    hipLaunchKernelGGL(prologue_conv_fwd, dim3(nconv), dim3(256), 0, st, p.dm, (const bf16*)x_bc,
                        conv_w, conv_b, (bf16*)x);
   });
   if (rc) return rc;
@@ -1047,7 +1048,7 @@ extern "C" int atomic_mamba2_proj_bwd(const atomic_mamba2_proj_args* a, const vo
   if (rc) return rc;
   const int ngrp = dm.L / (4 * kTileB);
   rc = L("prologue_conv_bwd", [&] {
-    hipLaunchKernelGGL((prologue_conv_bwd<kPlain, 128>), dim3((unsigned)((size_t)dm.B * ngrp * (dm.d / (64 * kCplB)))),
+    hipLaunchKernelGGL(prologue_conv_bwd, dim3((unsigned)((size_t)dm.B * ngrp * (dm.d / (64 * kCplB)))),
                        dim3(256), 0, st, dm, (const bf16*)x_bc, conv_w, conv_b, (const bf16*)dx, dxc, cpart);
   });
   if (rc) return rc;

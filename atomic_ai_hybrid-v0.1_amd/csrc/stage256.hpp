@@ -20,7 +20,8 @@ struct StageIn {
   int bf;  // 1: bf16, 0: fp32
 };
 // One dword load whatever the type (a bf16 element is one half of the aligned
-// dword that holds it), and selects: a branch on the type around each load
+// dword that holds it; the other half may lie outside the array, but never in
+// another page, and is not used), and selects: a branch on the type around each load
 // kept a loop's loads from being in flight together (eight of them in turn
 // were most of a GEMM tile's 28 us).
 __device__ __forceinline__ float ld(const StageIn& a, size_t i) {
