@@ -281,15 +281,15 @@ struct DhSeqLds {
 // bf16 dh loop of one (batch, head, VT columns), one workgroup per CU: waves
 // 0-7 compute (a dv_new tile and one 16-row block of dh each), the next NL load
 // the chunks (gdn2_seq.hpp), two bring dO in (it may be fp32 and row-strided, so
-// it passes through registers, to bf16) and one touches the lines of the chunk
-// four steps on.  As in the forward loop everything is computed transposed,
+// it passes through registers, to bf16) and one, when launched, touches the lines
+// of the chunk two steps on.  As in the forward loop everything is computed transposed,
 // and every product that does not need dv_new runs before the barrier that
 // waits for it.  Bound by the step's chain (1.2 us a chunk at 16 columns, 1.45
 // at 32 with the operands in L2; the former kernel, which staged through
 // registers, 1.5 and 2.6) and by HBM at 256 workgroups.
-// B4 T8192 H16, fp32 dO: 0.340 -> 0.297 ms; B8 T4096 H6 0.159 -> 0.127 ms; B1
-// T32768 H16 0.761 -> 0.607 ms (0.769 without the prefetch wave); K = 64, B2
-// T4096 H16 0.081 -> 0.060 ms.
+// Kernel times with an fp32 dO, former -> now: B4 T8192 H16 0.314 -> 0.245 ms; B8
+// T4096 H6 0.156 -> 0.118; B1 T32768 H16 0.748 -> 0.603; K = 64, B4 T4096 H16 0.099 ->
+// 0.079.
 // AL = false: a workspace that is not 16-byte aligned.
 template <typename TD, int C, int K, int V, int VT, int NL, bool AL = true>
 __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
@@ -314,7 +314,9 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
   unsigned char* sDv = lds + L::off_dv;
   // chunk of step i: NT - 1 - i; its buffers: i & 1
   if (wid == 8 + NL + 2) {
-    // ---------------- L2 prefetch, four chunks ahead; the V tiles of a head share an XCD and split its lines
+    // ---------------- L2 prefetch of the chunk that the loader waves request in this step; the V
+    // tiles of a head share an XCD and split its lines.  (Four chunks ahead the lines were gone
+    // again: B4 T8192 H16 fetched 1.53 times the bytes of the loaders alone, 0.266 -> 0.244 ms.)
     auto touch = [&](const void* p, int bytes) { touch_lines(p, bytes, NVT, vt, lds + L::off_pf); };
     auto pf = [&](int i) {
       if (i > last) return;
@@ -324,9 +326,8 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_bwd_dh(
       touch(ck.kg + (bh0 + n) * (C * K), C * K * 2);
       touch(ck.aqk + (bh0 + n) * (C * C), C * C * 2);
     };
-    pf(2); pf(3);
     bare_barrier();
-    for (int i = 0; i < dm.NT; ++i) { pf(i + 4); bare_barrier(); bare_barrier(); }
+    for (int i = 0; i < dm.NT; ++i) { pf(i + 2); bare_barrier(); bare_barrier(); }
     vm_wait<0>();  // nothing may still be on its way to this workgroup's LDS when it ends
     return;
   }

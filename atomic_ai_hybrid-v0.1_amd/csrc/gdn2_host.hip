@@ -218,12 +218,13 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
         return;
       }
       // The prefetch wave where the tiles of a head share an L2 (elsewhere each
-      // XCD gets only its share of the lines: B3 T4096 H21, 32 columns, 0.212 ms
-      // with it, 0.173 without), and with 32 columns only while the workgroups
-      // leave CUs idle, where latency bounds the step (B8 T4096 H6 with saves
-      // 0.155 ms with it, 0.168 without; B4 T4096 H16, 256 workgroups, 0.136 and
-      // 0.130).  With 16 columns it pays up to all 256 CUs (B1 T8192 H32: 0.159
-      // and 0.210 ms, with saves 0.193 and 0.278; B1 T32768 H16: 0.51 and 0.62).
+      // XCD gets only its share of the lines: B3 T4096 H21, 32 columns, 0.186 ms
+      // with it, 0.173 without; T2048, 12 heads 0.035 and 0.033).  There it hides
+      // latency with 16 columns (B1 T8192 H32: 0.156 ms with it, 0.208 without,
+      // with saves 0.187 and 0.279; B1 T32768 H16: 0.51 and 0.66) and with 32 while
+      // the workgroups leave CUs idle or store the saves (B8 T4096 H6 with saves
+      // 0.152 and 0.168; B4 T8192 H16 with saves 0.307 and 0.321; B4 T4096 H16, 256
+      // workgroups without saves, 0.132 and 0.131).
       const bool shared = gdn2_tiles_share_l2(bh);
       if (narrow) {
         const unsigned nwg = (unsigned)(bh * (V / 16));
@@ -232,7 +233,7 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
       } else {
         const unsigned nwg = (unsigned)(bh * (V / 32));
         hipLaunchKernelGGL((gdn2_fwd_state<C, K, V, 32, 4>), dim3(nwg),
-                           dim3(512 + 64 * (4 + ns + (shared && nwg < 256))), 0, st, p.dm, ck, h0, o, h_final, mode);
+                           dim3(512 + 64 * (4 + ns + (shared && (nwg < 256 || ns)))), 0, st, p.dm, ck, h0, o, h_final, mode);
       }
     } else {
       if (narrow)
@@ -292,16 +293,16 @@ static int gdn2_backward_impl(const Gdn2Plan& p, const void* q, const void* k, c
   const int bh = p.dm.B * p.dm.H;
   const unsigned nblk = (unsigned)p.bhn;
   // 16-column V tiles under the same condition as the forward state loop (B4
-  // T8192 H16 K = 128: 0.39 ms with 16, 0.30 with 32).  The prefetch wave too,
-  // except that at K = 128 it pays with 32 columns and a full chip as well (B4
-  // T8192 H16 0.264 ms with it, 0.278 without; B8 T4096 H24 0.402 and 0.424; at K =
-  // 64, B8 T4096 H16, 0.128 and 0.116).
+  // T8192 H16 K = 128: 0.39 ms with 16, 0.30 with 32).  The prefetch wave where
+  // tiles share an L2, with 16 columns (B1 T8192 H32: 0.170 ms with it, 0.231
+  // without) and with 32 at K = 128 (B4 T8192 H16 0.246 and 0.281), where a chunk
+  // is twice the bytes of K = 64 (B8 T4096 H12 0.103 and 0.096).
   rc = L("gdn2_bwd_dh", [&] {
     if constexpr (sizeof(T) == 2) {
       constexpr int NL = 2, NT0 = 512 + 64 * (NL + 2);
       const bool al = gdn2_aligned(ck), narrow = al && gdn2_narrow(bh, V);
       const unsigned nwg = (unsigned)(bh * (V / (narrow ? 16 : VT)));
-      const unsigned nthr = NT0 + 64 * (gdn2_tiles_share_l2(bh) && (narrow || K == 128 || nwg < 256));
+      const unsigned nthr = NT0 + 64 * (gdn2_tiles_share_l2(bh) && (narrow || K == 128));
       if (!al)  // as in the forward state loop
         hipLaunchKernelGGL((gdn2_bwd_dh<TD, C, K, V, VT, NL, false>), dim3(nwg), dim3(NT0), 0, st, p.dm, ck, gr,
                            (const TD*)dO, dh_final, dh0);
