@@ -634,8 +634,8 @@ struct StateLds {
 // bf16 state loop of one (batch, head, VT columns): waves 0-3 compute v_new
 // and the state, 4-7 o, the next NL load the chunks (see gdn2_seq.hpp), two more
 // store the saves (32 columns), and a last one, when launched, touches the lines
-// of the chunk kPrefetch steps on: it hides the memory latency that two chunks in
-// flight do not cover.
+// of the chunk kPrefetch steps on: it hides memory latency that the loaders'
+// two chunks in flight do not cover.
 // v_new and the state are computed transposed (columns of h as MFMA rows), so
 // a lane's four results are four consecutive columns of one row of the LDS
 // copies.  Bound by the step's chain of LDS reads, MFMAs and two barriers when
@@ -643,18 +643,20 @@ struct StateLds {
 // 128; the former kernel, in which every wave loaded, staged and computed,
 // 1.40 and 1.7), and by HBM with 256 workgroups and the saves.
 // Kernel times, former -> now: B1 T32768 H16 0.822 -> 0.508 ms, with saves 0.902
-// -> 0.618; B8 T4096 H6 with saves 0.172 -> 0.152; B4 T8192 H16 0.270 -> 0.231,
-// with saves 0.329 -> 0.307; K = 64 with saves, B2 T4096 H16 0.097 -> 0.070, B8
+// -> 0.618; B8 T4096 H6 with saves 0.172 -> 0.150; B4 T8192 H16 0.270 -> 0.231,
+// with saves 0.329 -> 0.297; K = 64 with saves, B2 T4096 H16 0.097 -> 0.070, B8
 // T4096 H16 0.135 -> 0.137.
 // The saves at 32 columns: as 64-byte row pieces by the o waves, inside their MFMA
 // chain, they took the same bytes 0.344 ms at B4 T8192 H16 (the pieces by waves of
-// their own 0.348), as whole rows 0.321, with the prefetch wave 0.307.  At 16
+// their own 0.348), as whole rows 0.321, with the prefetch wave 0.297.  At 16
 // columns latency bounds the step and more waves reading LDS lengthen it (B1
 // T32768 H16: 0.634 against 0.617), so there the o waves store them.
-// The prefetch distance: with four chunks the lines are partly gone again when the
-// loader waves come (B8 T4096 H6 with saves: 1.19 times the bytes, 0.155 ms), with
-// three 1.02 times and 0.152; two gain there (0.150) but not at 16 columns (B1
-// T32768 H16 with saves 0.616 at four, 0.618 at three, 0.623 at two).
+// The prefetch distance: lines touched too early are gone again when the loader
+// waves come.  32 columns, K = 128: two chunks (the one that the loaders request in
+// the same step; B4 T8192 H16 with saves 0.297 ms and the bytes of the loaders
+// alone; three chunks 1.3 times those and 0.307; B8 T4096 H6 0.150, three 0.152,
+// four 1.19 times and 0.155).  Else three (B8 T4096 H12 K = 64 with saves 0.100 ms, two
+// 0.105; 16 columns, B1 T32768 H16 with saves 0.618, two 0.623).
 // AL = false: per-chunk arrays that are not 16-byte aligned (a caller's own).
 template <int C, int K, int V, int VT, int NL, bool AL = true>
 __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_fwd_state(
@@ -665,7 +667,7 @@ __global__ __launch_bounds__(512 + 64 * (NL + 3)) void gdn2_fwd_state(
   __shared__ __attribute__((aligned(1024))) unsigned char lds[L::total];
   constexpr int NVT = V / VT, NTI = VT / 16, RB = K / 64, XK = K / 32, XC = C / 32, PK = K / 8;
   static_assert(C == 64 && K % 64 == 0, "four row blocks");
-  constexpr int kPrefetch = 3;
+  constexpr int kPrefetch = VT == 32 && K == 128 ? 2 : 3;
   int bh, vt;
   xcd_group_map(blockIdx.x, dm.B * dm.H, NVT, bh, vt);
   const int h = bh % dm.H, bb = bh / dm.H;

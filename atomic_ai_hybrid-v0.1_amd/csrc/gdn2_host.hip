@@ -223,8 +223,8 @@ static int gdn2_state_launch(const Gdn2Plan& p, const Gdn2Chunks<T>& ck, const f
       // latency with 16 columns (B1 T8192 H32: 0.156 ms with it, 0.208 without,
       // with saves 0.187 and 0.279; B1 T32768 H16: 0.51 and 0.66) and with 32 while
       // the workgroups leave CUs idle or store the saves (B8 T4096 H6 with saves
-      // 0.152 and 0.168; B4 T8192 H16 with saves 0.307 and 0.321; B4 T4096 H16, 256
-      // workgroups without saves, 0.132 and 0.131).
+      // 0.150 and 0.168; B4 T8192 H16 with saves 0.297 and 0.321; B4 T4096 H16, 256
+      // workgroups without saves and three chunks ahead, 0.132 and 0.131).
       const bool shared = gdn2_tiles_share_l2(bh);
       if (narrow) {
         const unsigned nwg = (unsigned)(bh * (V / 16));
